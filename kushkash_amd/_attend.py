@@ -1,0 +1,143 @@
+"""The prefill attention kernel (csrc/kush_attend.hip, include/kushkash_amd_attend.h): which inputs it takes,
+how a call is spread over the chip, and the call. Half-precision rows on the GPU, any batch and row strides,
+GQA, causal with the queries at the end of the keys or not, ragged rows packed end to end; forward only.
+Reference: the varlen flash attention of kushkash/vllm/backend.py:837-880."""
+from __future__ import annotations
+
+import ctypes
+import math
+from functools import lru_cache
+
+import torch
+
+from . import _lib
+
+_P, _I32, _I64, _F = ctypes.c_void_p, ctypes.c_int32, ctypes.c_int64, ctypes.c_float
+# head_dim, dtype, q, k, v, out, lse, strides, cu_q, cu_k, n_q, n_k, total_q, n_seqs, hkv, group, scale, causal,
+# out_f32, waves, chunk, part_o, part_ml, stream
+SIGNATURE = [_I32, _I32, _P, _P, _P, _P, _P, _P, _P, _P, _I32, _I32, _I64, _I32, _I32, _I32, _F, _I32, _I32, _I32,
+             _I32, _P, _P, _P]
+CUS = 256                        # MI355X compute units
+KEYS = 64                        # keys per tile
+PARTIAL_BYTES = 1 << 28          # at most this much scratch for split keys
+_Strides = ctypes.c_int64 * 15
+
+
+@lru_cache(None)
+def _entry():
+    fn = _lib.lib().kush_attend
+    fn.argtypes, fn.restype = SIGNATURE, ctypes.c_int32
+    return fn
+
+
+def _plain(*ts: torch.Tensor) -> bool:
+    """Whether the tensors are what a kernel can be handed: no subclass, no tracing or transform around
+    them, and no derivative asked for (the kernel has none)."""
+    if any(type(t) not in (torch.Tensor, torch.nn.Parameter) for t in ts):
+        return False
+    if torch.is_grad_enabled() and any(t.requires_grad for t in ts):
+        return False
+    return not (torch.compiler.is_compiling() or torch._C._functorch.peek_interpreter_stack() is not None
+                or torch._C._len_torch_dispatch_stack() or torch.autograd.forward_ad._current_level >= 0)
+
+
+def _row_strides(t: torch.Tensor, D: int) -> tuple[int, int, int]:
+    """(batch, row, head) strides of [.., rows, heads, D]; a dim of one entry counts as packed."""
+    st = [0 if t.dim() == 3 or t.shape[0] == 1 else t.stride(0), t.stride(-3), t.stride(-2)]
+    if t.shape[-3] == 1:
+        st[1] = D
+    if t.shape[-2] == 1:
+        st[2] = D
+    return tuple(st)
+
+
+def takes(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: float) -> bool:
+    """Whether the kernel takes q [B, T, Hq, D] (or packed [rows, Hq, D]) over k, v [B, N, Hk, D]: anything
+    else is the caller's other paths' (torch's flash kernel, fp32 products)."""
+    D = q.shape[-1]
+    if (not q.is_cuda or q.dtype not in (torch.bfloat16, torch.float16) or D not in (64, 128, 256)
+            or not (k.dtype == v.dtype == q.dtype and k.device == v.device == q.device)
+            or not (0.0 < scale < math.inf) or k.shape != v.shape or k.shape[-1] != D or q.dim() != k.dim()
+            or (q.dim() == 4 and q.shape[0] != k.shape[0]) or not _plain(q, k, v)):
+        return False
+    T, Hq, Hk = q.shape[-3], q.shape[-2], k.shape[-2]
+    if not q.numel() or not k.numel() or Hq % Hk or T * (Hq // Hk) > 1 << 22 or k.shape[-3] > 1 << 30:
+        return False
+    for t in (q, k, v):
+        st = _row_strides(t, D)
+        if t.stride(-1) != 1 or t.data_ptr() % 16 or any(s % 8 or s < 0 for s in st):
+            return False
+        if t is not q and not D <= st[1] <= 1 << 23:
+            return False
+    return True
+
+
+def plan(spans, group: int, hkv: int, D: int, total_q: int) -> tuple[int, int]:
+    """(waves, chunk) of a call whose sequences have (T, N, count) query rows and keys. A row tile is 32 waves
+    query rows (group heads of each token) of one kv head; 4 waves fill half a CU (a whole one at D 256, a
+    quarter at D 64), 8 a whole one.
+      8 waves  share each K / V tile among twice the rows: 1,031-1,045 us against 1,066-1,083 at 2,048 tokens x
+               4 heads over 34,816 keys, all of the chip's 256 row tiles of it busy to the end. With fewer or
+               shorter row tiles the last of them leave more of the chip idle than 4 waves do: 171 us against 146 for
+               two first prompts of 3,001 tokens, 293 against 264 for nine chunks over 8,000 keys.
+      chunk    split the keys of a row tile where the row tiles leave the chip idle, into as many parts as fill it
+               (256 tokens over 8,000 keys: 167 -> 67 us), or, where the longest would run on alone, into
+               halves (the nine chunks: 315 -> 264 us). Not below 24 tiles: the merge launch costs ~4 us, what 3 key
+               tiles cost (1,000 tokens over themselves: 27 us whole, 31-34 split)."""
+    longest = max(n for _, n, _ in spans)
+    bm = 128
+    if D <= 128 and longest >= 16384 and sum(c * (-(-t * group // 256)) for t, _, c in spans) * hkv >= CUS:
+        return 8, 0
+    tasks = units = 0
+    for t, n, c in spans:
+        tiles = -(-t * group // bm) * c
+        tasks += tiles
+        units += tiles * -(-(n - t // 2) // KEYS)
+    tasks, units = tasks * hkv, units * hkv
+    slots = CUS * {64: 4, 128: 2, 256: 1}[D]
+    nt = -(-longest // KEYS)
+    if nt < 24 or not tasks:
+        return 4, 0
+    if 2 * tasks <= slots:
+        chunk = -(-nt // (slots // tasks))
+    elif nt * slots > (1.2 if tasks > slots else 1.6) * units:
+        chunk = -(-max(2 * units // slots, nt) // 2)
+    else:
+        return 4, 0
+    row = total_q * hkv * group * (D + 2) * 4
+    chunk = max(chunk, 12, -(-nt * row // PARTIAL_BYTES))
+    return 4, chunk if chunk < nt else 0
+
+
+def attend(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: bool, scale: float, lse: bool = False,
+           cu: tuple | None = None, spans=None, out: torch.Tensor | None = None):
+    """Attention of inputs that takes() accepts: out in q's shape and type (the given one, its rows 16-byte
+    aligned, or a new one), or with lse the pair (out fp32, lse fp32 [.., Hq]). cu = (cu_q, cu_k, max_q, max_k)
+    and spans = [(T, N)] for packed rows: the offsets as int32 device tensors, the lengths on the host."""
+    D, Hq, Hk = q.shape[-1], q.shape[-2], k.shape[-2]
+    group = Hq // Hk
+    if cu is None:
+        seqs, n_q, n_k, total = q.shape[0], q.shape[1], k.shape[1], q.shape[0] * q.shape[1]
+        cq = ck = None
+        waves, chunk = plan(((n_q, n_k, seqs),), group, Hk, D, total)
+    else:
+        cq, ck, n_q, n_k = cu[0].data_ptr(), cu[1].data_ptr(), cu[2], cu[3]
+        seqs, total = len(spans), q.shape[0]
+        waves, chunk = plan([(t, n, 1) for t, n in spans], group, Hk, D, total)
+    dev = q.device
+    if out is None:
+        out = torch.empty(q.shape, dtype=torch.float32 if lse else q.dtype, device=dev)
+    logs = torch.empty(q.shape[:-1], dtype=torch.float32, device=dev) if lse else None
+    ls = _row_strides(logs.unsqueeze(-1), 1) if lse else (0, 0, 0)
+    strides = _Strides(*_row_strides(q, D), *_row_strides(k, D), *_row_strides(v, D), *_row_strides(out, D), *ls)
+    rows = -(-(-(-n_k // KEYS)) // chunk) * total * Hq if chunk else 0          # partial rows: every split's
+    part = torch.empty(rows * (D + 2), dtype=torch.float32, device=dev) if chunk else None
+    with torch.cuda.device(dev):
+        rc = _entry()(D, 1 if q.dtype == torch.float16 else 2, q.data_ptr(), k.data_ptr(), v.data_ptr(),
+                      out.data_ptr(), logs.data_ptr() if lse else None, ctypes.addressof(strides), cq, ck, n_q, n_k,
+                      total, seqs, Hk, group, scale, int(causal), int(lse), waves, chunk,
+                      part.data_ptr() if chunk else None, part.data_ptr() + rows * D * 4 if chunk else None,
+                      torch.cuda.current_stream(dev).cuda_stream)
+    if rc:
+        raise RuntimeError(f"kush_attend failed ({rc}): {(_lib.lib().kush_last_error() or b'').decode(errors='replace')}")
+    return (out, logs) if lse else out

@@ -5,11 +5,13 @@ unpack kernel; the serving engines' packed prefill, ragged_attention) and as the
 that path (history_attention, where they are dequantized by torch). Reference semantics:
 kushkash/_ops.py:254-285 (attention with log-sum-exp, merge), :309-339 (history attention).
 
-Two ways to attend a block: torch products in fp32 (the reference path, and any input the fused
-kernel does not take), or, where the caller asks for it (`fused`), torch's flash-attention kernel on
-the GPU for bf16 / fp16 inputs, which returns the log-sum-exp the merges need, takes the GQA head
-groups and aligns a causal block's queries with its last keys -- what the reference uses where its
-platform has it (_ops.py:254-276, vllm/backend.py:837-880). KUSHKASH_ATTN=fp32 keeps the products.
+Three ways to attend a block: torch products in fp32 (the reference path, and any input the fused
+kernels do not take), or, where the caller asks for it (`fused`), on the GPU for bf16 / fp16 inputs, this
+package's prefill attention kernel (_attend: it returns the log-sum-exp the merges need, takes the GQA
+head groups and any row strides, and aligns a causal block's queries with its last keys) or, for what
+that does not take (rows not 16-byte aligned, derivatives), torch's flash-attention kernel -- what the
+reference uses where its platform has it (_ops.py:254-276, vllm/backend.py:837-880). KUSHKASH_ATTN=fp32
+keeps the products.
 
 Memory: with the products, a block's score matrix [B, Hk, G*T, n] fp32 (and its exponentials) and its
 K / V in fp32 are what a block costs; the block length n is chosen so that they stay within
@@ -23,6 +25,7 @@ from functools import lru_cache
 
 import torch
 
+from . import _attend
 from ._records import PAGE, as_records, dequant_records
 
 
@@ -47,12 +50,17 @@ def fused_ok(q: torch.Tensor) -> bool:
 
 
 def _flash(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: bool, scale: float):
-    """attn_lse by torch's flash-attention kernel, or None where it refuses the shape. Without a mask
-    the q heads of a kv head are folded into its query rows (one kernel head per kv head); causal
-    blocks pass the head groups to the kernel, which aligns the queries with the last T keys."""
+    """attn_lse by the prefill attention kernel, by torch's flash-attention kernel for what that does not
+    take, or None where both refuse the input. torch's: without a mask the q heads of a kv head are folded
+    into its query rows (one kernel head per kv head); causal blocks pass the head groups to the kernel,
+    which aligns the queries with the last T keys."""
     B, Hq, T, D = q.shape
     Hk, N = k.shape[1], k.shape[2]
     g = Hq // Hk
+    rows = [x.transpose(1, 2) for x in (q, k, v)]
+    if _attend.takes(*rows, scale):
+        o, lse = _attend.attend(*rows, causal, scale, lse=True)
+        return o.transpose(1, 2), lse.transpose(1, 2)
     kt, vt = k.transpose(1, 2).contiguous(), v.transpose(1, 2).contiguous()           # [B, N, Hk, D]
     try:
         if causal:
@@ -143,23 +151,30 @@ def self_attention_blocks(q: torch.Tensor, k_new: torch.Tensor, v_new: torch.Ten
 
 
 def ragged_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, q_start: list, k_start: list, scale: float,
-                     block_bytes: int = 1 << 28, varlen: tuple | None = None) -> torch.Tensor:
+                     block_bytes: int = 1 << 28, varlen: tuple | None = None,
+                     out: torch.Tensor | None = None) -> torch.Tensor:
     """Causal attention of ragged rows packed end to end: row i's queries q[q_start[i]:q_start[i+1]]
     ([rows, Hq, D]) over its keys k, v[k_start[i]:k_start[i+1]] ([rows, Hk, D]), the queries being the
     last T of the row's N keys (query t sees keys j <= N - T + t: the serving engines' prefill
     convention). varlen = (cu_q, cu_k, max_q, max_k), the offsets as int32 device tensors: every row in
-    one launch of torch's flash-attention kernel (varlen form) where it takes q and no row is empty;
-    otherwise fp32 products per row, keys in blocks that keep each block's scores within block_bytes.
-    Returns q's shape and dtype."""
+    one call of the prefill attention kernel or torch's flash-attention kernel (varlen form) where they take
+    q and no row is empty; otherwise fp32 products per row, keys in blocks that keep each block's scores
+    within block_bytes. Returns q's shape and dtype, in out when given."""
     if (varlen is not None and fused_ok(q)
             and all(b > a for a, b in zip(q_start[:-1], q_start[1:]))):
         cu_q, cu_k, max_q, max_k = varlen
+        spans = [(b - a, d - c) for a, b, c, d in zip(q_start[:-1], q_start[1:], k_start[:-1], k_start[1:])]
+        if _attend.takes(q, k, v, scale) and all(n >= t for t, n in spans):
+            dst = out if out is not None and _attend.takes(out, k, v, scale) else None
+            o = _attend.attend(q, k, v, True, scale, cu=varlen, spans=spans, out=dst)
+            return o if out is None or dst is not None else out.copy_(o)
         try:
-            return torch.ops.aten._flash_attention_forward(q, k, v, cu_q, cu_k, max_q, max_k, 0.0, True, False,
-                                                           scale=scale)[0]
+            o = torch.ops.aten._flash_attention_forward(q, k, v, cu_q, cu_k, max_q, max_k, 0.0, True, False,
+                                                        scale=scale)[0]
+            return o if out is None else out.copy_(o)
         except RuntimeError:
             pass
-    out = q.new_empty(q.shape)
+    out = q.new_empty(q.shape) if out is None else out
     Hk, D = k.shape[1], k.shape[2]
     for i in range(len(q_start) - 1):
         a, b, c, d = q_start[i], q_start[i + 1], k_start[i], k_start[i + 1]
@@ -207,13 +222,40 @@ def history_attention(q: torch.Tensor, k_new: torch.Tensor, v_new: torch.Tensor,
     return acc[0].to(q.dtype)
 
 
+def _unpacked_rows(ops, k_new: torch.Tensor, v_new: torch.Tensor, cache: torch.Tensor, block_table: torch.Tensor,
+                   n_hist: int, tail_k: torch.Tensor, tail_idx: torch.Tensor, rot: bool):
+    """The n_hist cached tokens of every sequence and its new rows k_new, v_new [B, Hk, T, D] as K, V
+    [B, n_hist + T, Hk, D], by one launch of the unpack kernel."""
+    B, Hk, T, D = k_new.shape
+    dev, full, rows = k_new.device, n_hist // PAGE, n_hist + T
+
+    def first_rows(start: int, stop: int, step: int) -> torch.Tensor:      # rows start, start + step, .. of each sequence
+        r = torch.arange(start, stop, step, device=dev, dtype=torch.int32)
+        if B == 1:
+            return r
+        return (torch.arange(0, B * rows, rows, device=dev, dtype=torch.int32)[:, None] + r).view(-1)
+
+    new = [x.transpose(1, 2).reshape(B * T, Hk, D) for x in (k_new, v_new)]
+    kp, vp = (torch.empty(B, rows, Hk, D, dtype=ops.dtype, device=dev) for _ in range(2))
+    tail_blk = info = torch.zeros(0, dtype=torch.int32, device=dev)
+    if n_hist % PAGE:
+        tail_blk = block_table[:, full].contiguous()
+        first = first_rows(full * PAGE, full * PAGE + 1, 1)
+        info = torch.stack([first, torch.full_like(first, n_hist % PAGE), tail_idx[:B].to(torch.int32)], dim=1).view(-1)
+    ops.unpack(cache, block_table[:, :full].reshape(-1), first_rows(0, full * PAGE, PAGE), tail_blk, info, tail_k, *new,
+               first_rows(n_hist, rows, 1), kp.view(-1, Hk, D), vp.view(-1, Hk, D), rot)
+    return kp, vp
+
+
 def unpacked_history_attention(ops, q: torch.Tensor, k_new: torch.Tensor, v_new: torch.Tensor, cache: torch.Tensor,
                                block_table: torch.Tensor, n_hist: int, tail_k: torch.Tensor, tail_idx: torch.Tensor,
                                scale: float, rot: bool, block_bytes: int = 1 << 28) -> torch.Tensor:
     """history_attention on the GPU kernels: each block of history pages (all B sequences) is unpacked
     into K / V rows by one launch of the unpack kernel (Ops.unpack: fma(code, scale, bias) in fp32, one
     rounding to the cache dtype; rot rotates a rotated cache's rows back, so the attention runs on the
-    unrotated q and chunk), the partial page's K from the tail slots tail_idx. Shapes as
+    unrotated q and chunk), the partial page's K from the tail slots tail_idx. Where the prefill attention
+    kernel takes q, the history and the chunk are unpacked into one set of rows if block_bytes hold them, and
+    attended by one causal call; else each block is attended by itself and the blocks merged. Shapes as
     history_attention; returns [B, Hq, T, D] in q's dtype."""
     B, Hq, T, D = q.shape
     Hk = k_new.shape[1]
@@ -221,10 +263,18 @@ def unpacked_history_attention(ops, q: torch.Tensor, k_new: torch.Tensor, v_new:
     acc = None
     full = n_hist // PAGE
     r = n_hist - full * PAGE
+    key_bytes = 2 * B * Hk * D * (torch.finfo(dt).bits // 8)
+    kernel = T > 0 and q.dtype == dt and fused_ok(q) and _attend.takes(q.transpose(1, 2), *(
+        x.transpose(1, 2) for x in (k_new, v_new)), scale)
+    if kernel and n_hist and (n_hist + T) * key_bytes <= block_bytes:
+        kp, vp = _unpacked_rows(ops, k_new, v_new, cache, block_table, n_hist, tail_k, tail_idx, rot)
+        return _attend.attend(q.transpose(1, 2), kp, vp, True, scale).transpose(1, 2)
+    if kernel and not n_hist:
+        return _attend.attend(*(x.transpose(1, 2) for x in (q, k_new, v_new)), True, scale).transpose(1, 2)
     if n_hist:
         fused = fused_ok(q)
-        step = keys_per_block(q, Hk, 2 * B * Hk * D * (4 + torch.finfo(dt).bits // 8), block_bytes, PAGE,
-                              scores=not fused) // PAGE
+        step = keys_per_block(q, Hk, key_bytes if kernel else key_bytes + 8 * B * Hk * D, block_bytes, PAGE,
+                              scores=not fused) // PAGE                # (+ fp32 copies of K and V)
         none = torch.zeros(0, dtype=torch.int32, device=dev)
         empty = torch.zeros(0, Hk, D, dtype=dt, device=dev)
         p0 = 0

@@ -34,7 +34,7 @@ CPU_LIB = PKG / "libkushcpu.so"
 CPU_SOURCE = "kush_cpu.cpp"
 CPU_FLAGS = ["-O3", "-std=c++17", "-fPIC", "-shared", "-fopenmp", "-ffp-contract=off"]
 SOURCES = ("kush_capi.hip", "kush_write.hip", "kush_decode.hip", "kush_rotate.hip",
-           "kush_unpack.hip", "kush_decode_inst.hip")
+           "kush_unpack.hip", "kush_attend.hip", "kush_decode_inst.hip")
 # the decode kernel instantiations: one object per (input dtype, rot)
 DECODE_INST = [{"KUSH_INST_IN": t, "KUSH_INST_ROT": r} for t in ("float", "_Float16", "kush::bf16_t") for r in (0, 1)]
 
@@ -117,7 +117,7 @@ def source_digest(unit: str | None = None) -> str:
     h = hashlib.sha256()
     if unit is None:
         files = sorted((PKG / "csrc").glob("*.h")) + sorted((PKG / "csrc").glob("*.hip"))
-        files.append(ROOT / "include" / "kushkash_amd.h")
+        files += [ROOT / "include" / "kushkash_amd.h", ROOT / "include" / "kushkash_amd_attend.h"]
     else:
         seen: set = set()
         _includes(PKG / "csrc" / unit, seen)

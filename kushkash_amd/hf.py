@@ -24,6 +24,7 @@ from torch.nn.attention import SDPBackend, sdpa_kernel
 from transformers import AttentionInterface, AttentionMaskInterface
 from transformers.cache_utils import Cache, CacheLayerMixin
 
+from . import _attend
 from ._attention import self_attention_blocks
 from .cache import KushCache
 
@@ -133,13 +134,16 @@ class KushHFCache(Cache):
 def prompt_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: float,
                      block_bytes: int = 1 << 28) -> torch.Tensor:
     """Causal attention of a prompt over itself when nothing is cached yet: q [B, Hq, T, D], k, v
-    [B, Hkv, T, D] -> [B, Hq, T, D] in q's dtype (hf.py:122-129). Half-precision inputs go to torch's
-    fused attention, limited to its flash kernel (K / V expanded to the q heads); everything else, and
-    any input the flash kernel refuses, to fp32 products over blocks of keys whose memory stays within
-    block_bytes. torch's memory-efficient kernel is not allowed: on ROCm its dense and varlen forms are
+    [B, Hkv, T, D] -> [B, Hq, T, D] in q's dtype (hf.py:122-129). Half-precision inputs go to the prefill
+    attention kernel; what it does not take (rows not 16-byte aligned, derivatives) to torch's fused
+    attention, limited to its flash kernel (K / V expanded to the q heads); everything else, and any input
+    the flash kernel refuses, to fp32 products over blocks of keys whose memory stays within block_bytes. torch's memory-efficient kernel is not allowed: on ROCm its dense and varlen forms are
     the same kernel family, and its varlen form with a bottom-right causal mask has taken an
     illegal-address fault on this device. torch's half-precision math path (batched products over
     transposed views) is never taken either."""
+    rows = [x.transpose(1, 2) for x in (q, k, v)]
+    if _attend.takes(*rows, scale):
+        return _attend.attend(*rows, True, scale).transpose(1, 2)
     if q.dtype in (torch.float16, torch.bfloat16):
         g = q.shape[1] // k.shape[1]
         ke = k.repeat_interleave(g, 1) if g > 1 else k

@@ -1,0 +1,145 @@
+"""The prefill attention kernel (_attend.attend) against 64-bit attention at the edges of its tiles -- rows
+and keys of one, a tile, a tile and one, a ragged last tile -- for every head size, dtype, workgroup size and
+key split, with rows that are strided views; and what it leaves to the other paths."""
+import math
+
+import pytest
+import torch
+
+from kushkash_amd import _attend
+
+DEV = "cuda"
+# Relative 2-norm error of a correct kernel: the output's rounding and P's, u / sqrt(3) each for uniform rounding
+# errors at unit roundoff u = 2^-9 (bf16) / 2^-12 (fp16), P's at most that of a single key; twice their sum
+# leaves room for small samples.
+BOUND = {torch.bfloat16: 4 * 2.0 ** -9 / math.sqrt(3), torch.float16: 4 * 2.0 ** -12 / math.sqrt(3)}
+
+
+def _exact(q, k, v, causal, scale):
+    """Attention and log-sum-exp of one sequence, q [T, Hq, D], k, v [N, Hk, D], in 64 bits."""
+    T, N, G = q.shape[0], k.shape[0], q.shape[1] // k.shape[1]
+    qd, kd, vd = (x.double().cpu() for x in (q, k, v))
+    s = torch.stack([qd[:, h] @ kd[:, h // G].t() for h in range(q.shape[1])], 1) * scale            # [T, Hq, N]
+    if causal:
+        s.masked_fill_((torch.arange(N)[None] > torch.arange(T)[:, None] + N - T)[:, None], -math.inf)
+    p = torch.softmax(s, -1)
+    return torch.stack([p[:, h] @ vd[:, h // G] for h in range(q.shape[1])], 1), torch.logsumexp(s, -1)
+
+
+def _rel(a, b):
+    return ((a.double().cpu() - b).norm() / b.norm()).item()
+
+
+def _rows(shape, dt):
+    """Rows that are a slice of wider ones (16-byte aligned)."""
+    return torch.randn(*shape[:-2], shape[-2] + 1, shape[-1], device=DEV).to(dt)[..., 1:, :]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("D", [64, 128, 256])
+@pytest.mark.parametrize("T,N,Hk,G,causal", [
+    (1, 1, 1, 1, True), (1, 64, 2, 3, True), (32, 65, 1, 4, True), (33, 63, 2, 4, False), (65, 200, 1, 7, True),
+    (129, 130, 1, 2, True), (9, 1000, 2, 16, False), (300, 300, 1, 1, True)])
+def test_attention_at_tile_edges(D, dtype, T, N, Hk, G, causal, monkeypatch):
+    torch.manual_seed(T * N + D)
+    B, scale = 2, D ** -0.5
+    q, k, v = _rows((B, T, Hk * G, D), dtype), _rows((B, N, Hk, D), dtype) * 2, _rows((B, N, Hk, D), dtype)
+    assert _attend.takes(q, k, v, scale)
+    want = [_exact(q[b], k[b], v[b], causal, scale) for b in range(B)]
+    for waves, chunk in ((4, 0), (8, 0), (4, 1), (8, 3), (4, 5)):
+        print(D, dtype, T, N, Hk, G, causal, waves, chunk, flush=True)
+        monkeypatch.setattr(_attend, "plan", lambda *a: (waves, chunk))
+        out = _attend.attend(q, k, v, causal, scale)
+        out32, lse = _attend.attend(q, k, v, causal, scale, lse=True)
+        assert out.dtype == dtype and out.shape == q.shape and out32.dtype == torch.float32
+        for b in range(B):
+            assert _rel(out[b], want[b][0]) < BOUND[dtype]
+            assert _rel(out32[b], want[b][0]) < BOUND[dtype]
+            # log of a sum of weights each rounded to dtype (relative u) and fp32 scores (a few 1e-6)
+            assert (lse[b].double().cpu() - want[b][1]).abs().max() < BOUND[dtype]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("chunk", [0, 2])
+def test_ragged_rows(chunk, monkeypatch):
+    torch.manual_seed(3)
+    T, N = [5, 64, 1, 200, 17], [5, 300, 129, 200, 1017]
+    Hk, G, D, scale = 2, 4, 128, 0.11
+    q, k, v = (torch.randn(sum(n), h, D, device=DEV).bfloat16() for n, h in ((T, Hk * G), (N, Hk), (N, Hk)))
+    cu = [torch.tensor([0] + x, device=DEV).cumsum(0).to(torch.int32) for x in (T, N)]
+    monkeypatch.setattr(_attend, "plan", lambda *a: (4, chunk))
+    out = torch.empty_like(q)
+    got = _attend.attend(q, k, v, True, scale, cu=(*cu, max(T), max(N)), spans=list(zip(T, N)), out=out)
+    assert got is out
+    for i in range(len(T)):
+        a, b, c, d = *cu[0][i:i + 2].tolist(), *cu[1][i:i + 2].tolist()
+        assert _rel(out[a:b], _exact(q[a:b], k[c:d], v[c:d], True, scale)[0]) < BOUND[torch.bfloat16], i
+
+
+@pytest.mark.gpu
+def test_inputs_left_to_the_other_paths():
+    def rows(D=128, dt=torch.bfloat16):
+        return [torch.randn(1, 8, 2, D, device=DEV).to(dt) for _ in range(3)]
+
+    q, k, v = rows()
+    assert _attend.takes(q, k, v, 0.1)
+    assert not _attend.takes(*rows(96), 0.1) and not _attend.takes(*rows(dt=torch.float32), 0.1)
+    assert not any(_attend.takes(q, k, v, s) for s in (0.0, -1.0, math.inf, math.nan))
+    assert not _attend.takes(torch.randn(1, 8, 2, 129, device=DEV).bfloat16()[..., 1:], k, v, 0.1)    # misaligned
+    assert not _attend.takes(q, k.half(), v, 0.1) and not _attend.takes(q, k[..., :64], v[..., :64], 0.1)
+    assert not _attend.takes(q, k[:, :1].expand(1, 8, 2, 128), v, 0.1)                                # rows that repeat
+    assert not _attend.takes(q.requires_grad_(), k, v, 0.1)
+    with torch.no_grad():
+        assert _attend.takes(q, k, v, 0.1)
+
+
+@pytest.mark.parametrize("G", [1, 4, 7, 16])
+def test_the_plan_covers_the_keys_and_bounds_its_scratch(G):
+    """Whatever the shape: 4 or 8 waves, a split (if any) of at least 12 key tiles that leaves more than one
+    part, within the scratch bound, and no split where the row tiles fill the chip evenly."""
+    for D in (64, 128, 256):
+        for hkv in (1, 8):
+            for T, N, c in ((1, 1, 1), (16, 8016, 1), (256, 8256, 4), (2048, 34816, 1), (3001, 3001, 2), (1, 200000, 64)):
+                waves, chunk = _attend.plan(((T, N, c),), G, hkv, D, T * c)
+                nt = -(-N // 64)
+                assert waves in ((4, 8) if D < 256 else (4,)) and (chunk == 0 or 12 <= chunk < nt)
+                if chunk:
+                    assert -(-nt // chunk) * T * c * hkv * G * (D + 2) * 4 <= 2 * _attend.PARTIAL_BYTES
+    assert _attend.plan(((3001, 3001, 2),), 7, 4, 128, 6002) == (4, 0)
+    assert _attend.plan(((2048, 34816, 1),), 4, 8, 128, 2048) == (8, 0)
+
+
+def test_kernels_keep_their_wait_states(tmp_path):
+    """On the assembly: every read or overwrite of a 32x32x16 MFMA's result waits, on every control-flow path,
+    the 12 states that the compiler keeps in straight-line code (a branch join once broke this in the
+    decode), and m0 is only the LDS DMA's base, one wait state ahead of its load."""
+    import re
+    import shutil
+    import subprocess
+    from pathlib import Path
+
+    import test_isa
+    from kushkash_amd.build import FLAGS, ROOT
+    hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+    if not Path(hipcc).exists():
+        pytest.skip("hipcc not available")
+    subprocess.run([hipcc, *(f for f in FLAGS if f not in ("-shared", "-fPIC")), f"-I{ROOT / 'include'}", "-S",
+                    "--cuda-device-only", str(ROOT / "kushkash_amd/csrc/kush_attend.hip"), "-o",
+                    str(tmp_path / "a.s")], check=True, capture_output=True)
+    text = (tmp_path / "a.s").read_text().replace("13attend_kernel", "13decode_kernel")     # as kernels() finds them
+    found = test_isa.kernels(text)
+    assert len(found) == 10                                                # 3 head sizes x 2 dtypes, 8 waves for two
+    need = dict(test_isa.MFMA_WAIT, v_mfma_f32_32x32x16_bf16=12, v_mfma_f32_32x32x16_f16=12)
+    for name, lines in found.items():
+        saved = dict(test_isa.MFMA_WAIT)
+        test_isa.MFMA_WAIT.update(need)
+        try:
+            assert not test_isa.mfma_short_paths(lines), name
+        finally:
+            test_isa.MFMA_WAIT.clear()
+            test_isa.MFMA_WAIT.update(saved)
+        live = [l for l in lines if l]
+        for i, ins in enumerate(live):
+            if "m0" in ins:
+                assert re.match(r"s_mov_b32 m0, s\d+$", ins) and live[i + 1] == "s_nop 0" and live[i + 2].endswith(" lds"), ins
