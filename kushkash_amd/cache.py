@@ -16,9 +16,9 @@ of one page touch neighbouring records), the table never changes once written, a
 only appends blocks: the pool is reallocated with the old blocks as its prefix.
 
 Rotation. With rotation on (rotate=, KUSHKASH_ROTATE; on for 4-bit by default) the records and the
-tail hold K H and V H for the Hadamard matrix H: K, V and q are rotated on the way in and the
-decode output on the way out, by a torch product (the reference's rotation) or, with
-rotate_in_kernels=True, inside the write, append and decode kernels. Every public method takes and
+tail hold K H and V H for the Hadamard matrix H: K and V are rotated on the way in by a torch product (the
+reference's rotation) or, with rotate_in_kernels=True, inside the write and append kernels; q and the decode
+output inside the decode kernel (by torch products on the CPU). Every public method takes and
 returns unrotated tensors.
 """
 from __future__ import annotations
@@ -218,21 +218,31 @@ class KushCache:
         return self._decode(layer, q, token)
 
     def _decode(self, layer: int, q: torch.Tensor, token=None) -> torch.Tensor:
-        qk = self._inward(q).contiguous()
+        # A rotated cache's q and output are rotated inside the decode launch on the GPU, also where the
+        # rows it stores are rotated by the product (the rotations agree to fp32 rounding, and the output is
+        # rounded once instead of twice): one launch for the nine of q's and the output's conversions,
+        # products and scalings around it (4 sequences of 1,000 tokens, fp16: 96 -> 19 us a pass). The launch would
+        # rotate a token's rows too, so product-rotated ones are appended by a launch of their own.
+        rot = self.rot is not None and self.gpu
+        qk = (q.to(self.kdtype) if rot else self._inward(q)).contiguous()
         out = torch.empty_like(qk)
         pages = (self._capacity if self._splits else self._tokens[layer]) // PAGE
         splits = self._splits or self.ops.splits(self.B, self.H, pages)
         self._ensure_work(splits)
-        kw = {"rot": True} if self.krot else {}
+        kw = {"rot": True} if rot else {}
         if self.gpu:                                     # waves by the cached length (the table is wider)
             kw["waves"] = self.ops.waves(self.B, self.H, splits, pages)
-        args = (self.pool[layer], self.block_table, self.seq_lens[layer], self.tail_idx, self.tail_k[layer],
-                self.scale, splits, self._work)
+        dst = (self.pool[layer], self.block_table)
+        lens = (self.seq_lens[layer], self.tail_idx)
+        args = (*dst, *lens, self.tail_k[layer], self.scale, splits, self._work)
+        if token is not None and rot and not self.krot:
+            self.ops.append(*token, *lens, *dst, self.tail_k[layer], -1, False)
+            token = None
         if token is None:
             self.ops.decode(qk, out, *args, **kw)
         else:
             self.ops.append_decode(token[0], token[1], qk, out, *args, **kw)
-        return self._outward(out)
+        return out.to(self.dtype) if rot else self._outward(out)
 
     def attend_chunk(self, layer: int, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
                      block_bytes: int = 1 << 28) -> torch.Tensor:
