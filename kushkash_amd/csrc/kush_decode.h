@@ -21,14 +21,14 @@
 //      accumulates O^T += V^T . P'^T on MFMA, with P' = fp16(e * v_scale); -HALF * sum P' comes
 //      from one MFMA and the V bias sum e * v_bias stays in fp32.
 // The partial last page takes exact fp32 K . q scores from the tail (spread over all waves) and V
-// rows from its record. A rotated cache (ROT) gets q rotated by the canonical Walsh-Hadamard
-// transform on load (rows of the chunk's heads in the butterfly layout, through LDS) and the output
-// rotated back before its one rounding; split partials stay unrotated. With app_k (the fused append
-// + decode), the workgroup that reads the new token's page first appends the token (row s of app_k /
-// app_v at position seq_lens[s] - 1): K to the tail, V into its record row, the K page quantized
-// when the token completes it -- the page quantizer of kush_page.h over the idle ring LDS. The waves (and streams) merge through the idle ring at the end; with
-// split-K, partials are published write-through and the last workgroup of a (sequence, kv head)
-// merges them in the same launch.
+// rows from its record. A rotated cache (ROT) gets q rotated by the Walsh-Hadamard transform on load (on the
+// matrix cores for 16-bit q, rotate_q; an fp32 q in the canonical order through LDS) and the output rotated back
+// before its one rounding; split partials stay unrotated. With app_k (the fused append + decode), the
+// workgroup that reads the new token's page appends the token (row s of app_k / app_v at position
+// seq_lens[s] - 1): K to the tail, V into its record row by one wave behind the first page loads (NewToken), or,
+// when the token completes its page, ahead of them, the K page quantized by the page quantizer of kush_page.h over
+// the idle ring LDS. The waves (and streams) merge through the idle ring at the end; with split-K, partials
+// are published write-through and the last workgroup of a (sequence, kv head) merges them in the same launch.
 //
 // MFMA 16x16x32 f16 operand layout used throughout (lane l, r = l % 16, q = l / 16):
 //   A: row r, 8 contraction slots of lane group q;  B: column r, the same 8 slots;
@@ -93,6 +93,7 @@ struct TimelineMarks {
 #endif
 
 typedef _Float16 h4v __attribute__((ext_vector_type(4)));
+typedef __bf16 bh8 __attribute__((ext_vector_type(8)));
 
 __device__ __forceinline__ f4 mfma16(h8 a, h8 b, f4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0); }
 
@@ -257,17 +258,34 @@ __device__ __forceinline__ v2i gather_vt(const uint8_t* slot, int ct, int lane) 
     return __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i*)(src));
 }
 
+// V columns gathered ahead of a page pair's softmax: with one wave per SIMD nothing else covers an LDS read's
+// latency, and the compiler, short of registers, read the columns one by one with a full wait behind each.
+// As many as fit the 256 registers beside the loop's own: 4 columns of a pair (16 registers) at D <= 128, 2 of its
+// int8 codes, none with a third pair or a split's folded state beside those, nor at D 256.
+template <int D, int BITS, int DEP, bool WS>
+constexpr int vpre() {
+    return D == 256 || DEP == 3 || (D == 128 && BITS == 8 && WS) ? 0 : (D == 128 && BITS == 8 ? 2 : 4);
+}
+
 // Softmax update over NP staged pages at once and their PV accumulation from the staged V codes.
 // Scores in log2 units are x = a s[p][j] + b[p] (a > 0) for tokens tok(q, j); masked tokens carry
 // s = -inf. o accumulates in units of 2^-24 (subnormal codes; int4 high-nibble tiles, o[D/32 ..],
 // in units of 2^-20); with P' = fp16(e vs) a page adds sum P' n (MFMA), -HALF sum P' (MFMA into
 // vacc, units of 2^-24) and sum e vb (vb_run), i.e. sum e (vs' c + vb) with vs' = P' / e.
-template <int D, int BITS, int NP>
+template <int D, int BITS, int NP, int VPRE>
 __device__ __forceinline__ void consume_pages(const uint8_t* const (&slot)[NP], f4 (&o)[D / 16], f4& vacc,
                                               const float (&sv)[NP][8], float a, const float (&b)[NP],
                                               float& m_run, float& l_run, float& vb_run, int lane) {
     using F = Fmt<D, BITS>;
     const int q = lane >> 4;
+    // the first V columns, gathered ahead of the softmax, which covers their LDS latency (vpre)
+    constexpr int NCOL = BITS == 4 ? D / 32 : D / 16, PF = NCOL < VPRE ? NCOL : VPRE;
+    v2i wv[PF > 0 ? PF : 1][NP];
+#pragma unroll
+    for (int ct = 0; ct < PF; ++ct)
+#pragma unroll
+        for (int p = 0; p < NP; ++p) wv[ct][p] = gather_vt<D, BITS>(slot[p], ct, lane);
+    if constexpr (PF > 0) asm volatile("" ::: "memory");      // not sunk below this point
     float pm = -__builtin_inff();
 #pragma unroll
     for (int p = 0; p < NP; ++p) {
@@ -313,21 +331,23 @@ __device__ __forceinline__ void consume_pages(const uint8_t* const (&slot)[NP], 
         vacc *= corr;
     }
 
-    constexpr int NCOL = BITS == 4 ? D / 32 : D / 16;
 #pragma unroll
-    for (int ct = 0; ct < NCOL; ++ct)
+    for (int ct = 0; ct < NCOL; ++ct) {
+        v2i w[NP];
+#pragma unroll
+        for (int p = 0; p < NP; ++p) w[p] = ct < PF ? wv[ct][p] : gather_vt<D, BITS>(slot[p], ct, lane);
 #pragma unroll
         for (int p = 0; p < NP; ++p) {
-            const v2i w = gather_vt<D, BITS>(slot[p], ct, lane);
             if constexpr (BITS == 4) {
                 h8 lo, hi;
-                v_codes4((uint32_t)w[0], (uint32_t)w[1], lo, hi);
+                v_codes4((uint32_t)w[p][0], (uint32_t)w[p][1], lo, hi);
                 o[ct] = mfma16(lo, pw[p], o[ct]);
                 o[ct + D / 32] = mfma16(hi, pw[p], o[ct + D / 32]);
             } else {
-                o[ct] = mfma16(int8_sub((uint32_t)w[0], (uint32_t)w[1]), pw[p], o[ct]);
+                o[ct] = mfma16(int8_sub((uint32_t)w[p][0], (uint32_t)w[p][1]), pw[p], o[ct]);
             }
         }
+    }
     // -HALF sum P' per head: A rows all -HALF 2^-24 (fp16 bits 0x8000 | HALF, exact)
     const _Float16 nh = __builtin_bit_cast(_Float16, (uint16_t)(0x8000u | (uint32_t)F::HALF));
     const h8 neg_half = h8{nh, nh, nh, nh, nh, nh, nh, nh};
@@ -407,6 +427,7 @@ __device__ __forceinline__ void pair_scores(const uint8_t* s0, const h8 (&qa)[D 
 #pragma unroll
     for (int p = 0; p < 2; ++p) sacc[p][0] = sacc[p][1] = f4{0.0f, 0.0f, 0.0f, 0.0f};
     f4 bacc = f4{0.0f, 0.0f, 0.0f, 0.0f};
+    u4 kw[2][2];                                      // int8: the code chunks of two K-steps
 #pragma unroll
     for (int kk = 0; kk < KSTEPS; ++kk) {
         const int d0 = kdim<D, BITS>(kk, q, 0);
@@ -418,13 +439,14 @@ __device__ __forceinline__ void pair_scores(const uint8_t* s0, const h8 (&qa)[D 
                 // code bytes of row 16 tt + r16 for this K-step, from the swizzled slot
                 const int row = 16 * tt + r16;
                 const int byte = q * KBYTES + 8 * (BITS == 4 ? kk >> 1 : kk);
-                const u2 wv = *reinterpret_cast<const u2*>(sl[p] + slot_chunk<D, BITS>(row, byte / 16) + byte % 16);
                 if constexpr (BITS == 4) {
+                    const u2 wv = *reinterpret_cast<const u2*>(sl[p] + slot_chunk<D, BITS>(row, byte / 16) + byte % 16);
                     h8 lo, hi;
                     k_codes4(wv[0], wv[1], lo, hi);
                     a[tt] = (kk & 1) ? hi : lo;
-                } else {
-                    a[tt] = int8_sub(wv[0], wv[1]);
+                } else {                                         // a 16-byte chunk holds two K-steps
+                    if (kk % 2 == 0) kw[p][tt] = *reinterpret_cast<const u4*>(sl[p] + slot_chunk<D, BITS>(row, byte / 16));
+                    a[tt] = int8_sub(kw[p][tt][2 * (kk & 1)], kw[p][tt][2 * (kk & 1) + 1]);
                 }
             }
             const h8 ks8 = *reinterpret_cast<const h8*>(sl[p] + F::OFF_KS + 2 * d0);
@@ -481,6 +503,7 @@ __device__ __forceinline__ void pair_scores2(const uint8_t* s0, const h8 (&qa)[D
 #pragma unroll
     for (int p = 0; p < 2; ++p) sacc[p][0] = sacc[p][1] = f4{0.0f, 0.0f, 0.0f, 0.0f};
     f4 bacc = f4{0.0f, 0.0f, 0.0f, 0.0f};
+    u4 kw[2][2];                                      // int8: the code chunks of two K-steps
 #pragma unroll
     for (int kk = 0; kk < KSTEPS; ++kk) {
         const int d0 = kdim<D, BITS>(kk, q, 0);
@@ -499,13 +522,16 @@ __device__ __forceinline__ void pair_scores2(const uint8_t* s0, const h8 (&qa)[D
             for (int tt = 0; tt < 2; ++tt) {
                 const int row = 16 * tt + r16;
                 const int byte = q * KBYTES + 8 * (BITS == 4 ? kk >> 1 : kk);
-                const u2 wv = *reinterpret_cast<const u2*>(sl[p] + slot_chunk<D, BITS>(row, byte / 16) + byte % 16);
                 if constexpr (BITS == 4) {
+                    const u2 wv = *reinterpret_cast<const u2*>(sl[p] + slot_chunk<D, BITS>(row, byte / 16) + byte % 16);
                     h8 lo, hi;
                     k_codes4(wv[0], wv[1], lo, hi);
                     a[tt] = (kk & 1) ? hi : lo;
                 } else {
-                    a[tt] = int8_sub(wv[0], wv[1]);
+                    // a 16-byte chunk holds two K-steps: read whole (left to itself the compiler merged some of
+                    // these reads across rows instead, by how its code around the loop fell: 0.5 % of a decode)
+                    if (kk % 2 == 0) kw[p][tt] = *reinterpret_cast<const u4*>(sl[p] + slot_chunk<D, BITS>(row, byte / 16));
+                    a[tt] = int8_sub(kw[p][tt][2 * (kk & 1)], kw[p][tt][2 * (kk & 1) + 1]);
                 }
             }
             sacc[p][0] = mfma16(a[0], qp, sacc[p][0]);
@@ -527,12 +553,20 @@ __device__ __forceinline__ void pair_scores2(const uint8_t* s0, const h8 (&qa)[D
 // sv = -inf; a column may be masked whole) and the PV accumulation of page A (at s0) into columns
 // 0-7 and page B (at s0 + ds) into columns 8-15: each MFMA takes P' with the other stream's
 // columns zeroed. Units as in consume_pages.
-template <int D, int BITS>
+template <int D, int BITS, int VPRE>
 __device__ __forceinline__ void consume2(const uint8_t* s0, int ds, f4 (&o)[D / 16], f4& vacc, const float (&sv)[8],
                                          float a, float kx, float& m_run, float& l_run, float& vb_run, int lane) {
     using F = Fmt<D, BITS>;
     const int r16 = lane & 15, q = lane >> 4, st = r16 >> 3;
     const uint8_t* const mine = s0 + st * ds;
+    constexpr int NCOL = BITS == 4 ? D / 32 : D / 16, PF = NCOL < VPRE ? NCOL : VPRE;
+    v2i wv[PF > 0 ? PF : 1][2];                                                // as in consume_pages
+#pragma unroll
+    for (int ct = 0; ct < PF; ++ct) {
+        wv[ct][0] = gather_vt<D, BITS>(s0, ct, lane);
+        wv[ct][1] = gather_vt<D, BITS>(s0 + ds, ct, lane);
+    }
+    if constexpr (PF > 0) asm volatile("" ::: "memory");
     float pm = sv[0];
 #pragma unroll
     for (int j = 1; j < 8; ++j) pm = __builtin_fmaxf(pm, sv[j]);
@@ -575,11 +609,10 @@ __device__ __forceinline__ void consume2(const uint8_t* s0, int ds, f4 (&o)[D / 
         vacc *= corr;
     }
 
-    constexpr int NCOL = BITS == 4 ? D / 32 : D / 16;
 #pragma unroll
     for (int ct = 0; ct < NCOL; ++ct) {
-        const v2i wa = gather_vt<D, BITS>(s0, ct, lane);
-        const v2i wb = gather_vt<D, BITS>(s0 + ds, ct, lane);
+        const v2i wa = ct < PF ? wv[ct][0] : gather_vt<D, BITS>(s0, ct, lane);
+        const v2i wb = ct < PF ? wv[ct][1] : gather_vt<D, BITS>(s0 + ds, ct, lane);
         if constexpr (BITS == 4) {
             h8 lo, hi;
             v_codes4((uint32_t)wa[0], (uint32_t)wa[1], lo, hi);
@@ -606,7 +639,7 @@ constexpr int WIN = 1024;
 // waves' softmax state and the split-K flag in the second.
 template <int D, int BITS, int NW>
 constexpr int decode_lds_bytes() {
-    return 4 * NW * Ring<D, BITS>::SLOT + 4 * WIN + 16;
+    return 4 * NW * Ring<D, BITS>::SLOT + 4 * WIN + 5 * D + 48;      // the new token's copies: at most 5 D + 16 bytes
 }
 
 template <int D, int BITS, int NW>
@@ -639,18 +672,20 @@ struct Packed {
     // zero at first: set() of a half-width element keeps the other half of its word, which must
     // then be a defined value (an uninitialized one lets the optimizer fold the word away)
     uint32_t wd[WORDS] = {};
-    __device__ __forceinline__ void load(const IN* p) {          // p aligned to min(16, BYTES)
-        if constexpr (BYTES % 16 == 0) {
+    // elements [n R, (n + 1) R) from p, R = min(N, 8) (p aligned to min(16, R sizeof(IN)) bytes; n a constant)
+    static constexpr int R = N < 8 ? N : 8, RW = R * (int)sizeof(IN) / 4;
+    __device__ __forceinline__ void load_run(int n, const IN* p) {
+        if constexpr (RW % 4 == 0) {
 #pragma unroll
-            for (int i = 0; i < BYTES / 16; ++i) {
+            for (int i = 0; i < RW / 4; ++i) {
                 const u4 v = reinterpret_cast<const u4*>(p)[i];
 #pragma unroll
-                for (int j = 0; j < 4; ++j) wd[4 * i + j] = v[j];
+                for (int j = 0; j < 4; ++j) wd[n * RW + 4 * i + j] = v[j];
             }
         } else {
             const u2 v = *reinterpret_cast<const u2*>(p);
-            wd[0] = v[0];
-            wd[1] = v[1];
+            wd[n * RW] = v[0];
+            wd[n * RW + 1] = v[1];
         }
     }
     __device__ __forceinline__ float get(int k) const {          // k a constant after unrolling
@@ -671,31 +706,170 @@ struct Packed {
     }
 };
 
-// Rows r < n of an fp32 staging area [.][D] in LDS rotated back by the canonical Walsh-Hadamard
-// transform and rounded once into out (row stride D), by THREADS threads: D / 16 lanes per row in the
-// butterfly layout (a row's lanes iterate together).
-template <int D, typename IN, int THREADS>
-__device__ __forceinline__ void store_rotated(IN* __restrict__ out, const float* stage, int n, bool vec) {
-    constexpr int CG = D / 16, RP = THREADS / CG;
-    static_assert(THREADS % CG == 0, "whole rows per pass");
-    const int c = (int)threadIdx.x % CG;
-    for (int r = (int)threadIdx.x / CG; r < n; r += RP) {
-        float x[16];
+// E consecutive elements at p as one access (p aligned to their size)
+template <typename IN, int E>
+struct alignas(E * sizeof(IN)) Lanes {
+    IN v[E];
+};
+
+// Rows r, r + NR .. of an fp32 staging area [.][D] in LDS rotated back by the canonical Walsh-Hadamard transform
+// and rounded once into out (row stride D), N of them by the calling wave, their chains interleaved.
+template <int D, typename IN, int N, int NR>
+__device__ __forceinline__ void store_rotated_rows(IN* __restrict__ out, const float* stage, int r, int lane, bool vec) {
+    constexpr int E = D / WAVE;
+    float x[N][E];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            x[j] = stage[r * D + 8 * c + j];
-            x[8 + j] = stage[r * D + D / 2 + 8 * c + j];
-        }
-        fwht_runs<D>(x, c);
+    for (int i = 0; i < N; ++i)
+#pragma unroll
+        for (int e = 0; e < E; ++e) x[i][e] = stage[(r + i * NR) * D + E * lane + e];
+#pragma unroll
+    for (int i = 0; i < N; ++i) fwht_wave<D>(x[i], lane);
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        IN* const dst = out + (int64_t)(r + i * NR) * D + E * lane;
+        Lanes<IN, E> y;
+#pragma unroll
+        for (int e = 0; e < E; ++e) y.v[e] = store_rounded<IN>(x[i][e]);
         if (vec) {
-            put8<true>(out + (int64_t)r * D + 8 * c, x);
-            put8<true>(out + (int64_t)r * D + D / 2 + 8 * c, x + 8);
+            *reinterpret_cast<Lanes<IN, E>*>(dst) = y;
         } else {
-            put8<false>(out + (int64_t)r * D + 8 * c, x);
-            put8<false>(out + (int64_t)r * D + D / 2 + 8 * c, x + 8);
+#pragma unroll
+            for (int e = 0; e < E; ++e) dst[e] = y.v[e];
         }
     }
 }
+
+// The staged rows r < n, a wave per row.
+template <int D, typename IN, int THREADS>
+__device__ __forceinline__ void store_rotated(IN* __restrict__ out, const float* stage, int n, bool vec) {
+    constexpr int NR = THREADS / WAVE;
+    const int lane = (int)threadIdx.x % WAVE;
+    int r = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+    for (; r + 3 * NR < n; r += 4 * NR) store_rotated_rows<D, IN, 4, NR>(out, stage, r, lane, vec);
+    for (; r + NR < n; r += 2 * NR) store_rotated_rows<D, IN, 2, NR>(out, stage, r, lane, vec);
+    if (r < n) store_rotated_rows<D, IN, 1, NR>(out, stage, r, lane, vec);
+}
+
+// q heads rotated on the matrix cores: qv[kk][j] = dim kdim(kk, q, j) of H x, rounded to IN, for this lane's column
+// from qraw[kk] = the dims kdim(kk, q, 0 .. 7) of x: the layout q is loaded and used in. Those dims are three
+// disjoint groups of index bits (j, lane group, kk), so H = H_8 (x) H_4 (x) H_KS: one MFMA per K-step and row half
+// sums over j and the lane groups with signs +-1 (exact products, fp32 sums; output row 4 q' + i of half hf
+// stands for j = 4 hf + i of lane group q'), and a butterfly over the K-steps in registers does the rest. No LDS
+// and no barrier, where the rotation through LDS put two of each before the second page pair.
+template <int D, typename IN>
+__device__ __forceinline__ void rotate_q(const u4 (&qraw)[D / 32], float (&qv)[D / 32][8], int lane) {
+    constexpr int KS = D / 32;
+    constexpr bool HALF16 = std::is_same<IN, _Float16>::value;
+    const int r = lane & 15, g = (r >> 2) & (lane >> 4);
+    const uint32_t both = 0x80008000u;
+    // sign of slot j of lane group q in row r: parity of (j & row's j) and of (q & row's lane group)
+    uint32_t one = HALF16 ? 0x3C003C00u : 0x3F803F80u;
+    one ^= ((g ^ (g >> 1)) & 1) ? both : 0u;
+    one ^= (r & 1) ? 0x80000000u : 0u;
+    const uint32_t two = one ^ ((r & 2) ? both : 0u);
+    const u4 a[2] = {u4{one, two, one, two}, u4{one, two, one ^ both, two ^ both}};
+    f4 t[KS][2];
+#pragma unroll
+    for (int kk = 0; kk < KS; ++kk)
+#pragma unroll
+        for (int hf = 0; hf < 2; ++hf) {
+            const f4 zero = f4{0.0f, 0.0f, 0.0f, 0.0f};
+            if constexpr (HALF16)
+                t[kk][hf] = mfma16(__builtin_bit_cast(h8, a[hf]), __builtin_bit_cast(h8, qraw[kk]), zero);
+            else
+                t[kk][hf] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bh8, a[hf]),
+                                                                    __builtin_bit_cast(bh8, qraw[kk]), zero, 0, 0, 0);
+        }
+#pragma unroll
+    for (int h = 1; h < KS; h <<= 1)
+#pragma unroll
+        for (int kk = 0; kk < KS; ++kk) {
+            if (kk & h) continue;
+#pragma unroll
+            for (int hf = 0; hf < 2; ++hf) {
+                const f4 x = t[kk][hf], y = t[kk + h][hf];
+                t[kk][hf] = x + y;
+                t[kk + h][hf] = x - y;
+            }
+        }
+    const float sc = fwht_scale<D>();
+#pragma unroll
+    for (int kk = 0; kk < KS; ++kk)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) qv[kk][j] = to_f32(store_rounded<IN>(t[kk][j >> 2][j & 3] * sc));
+}
+
+// The fused append's token, for a page that it does not complete: one wave holds its K and V rows (lane l the
+// D / 64 dims from l D / 64), rotates them when the cache does, and stores the K row into the tail and the
+// quantized V row into the record -- page_task's arithmetic, so its bytes -- with a copy of both in LDS. The
+// workgroup's own use of the row (its exact score, its V codes) takes those copies, so nothing in the launch
+// waits for the stores, and the page loop starts without the append.
+template <int D, int BITS, typename IN>
+struct NewToken {
+    using F = Fmt<D, BITS>;
+    static constexpr int E = D / WAVE;
+    Lanes<IN, E> k, v;
+    __device__ __forceinline__ void load(const IN* krow, const IN* vrow, int lane) {
+        k = *reinterpret_cast<const Lanes<IN, E>*>(krow + E * lane);
+        v = *reinterpret_cast<const Lanes<IN, E>*>(vrow + E * lane);
+    }
+    // tail: the token's row of the K tail; rec: the page's record, the token in row slot; lds: the copies (K row,
+    // V codes, then the V scale and bias as two fp16)
+    template <bool ROT>
+    __device__ __forceinline__ void store(IN* tail, uint8_t* rec, int slot, uint8_t* lds, int lane) {
+        float x[E];
+        if constexpr (ROT) {
+#pragma unroll
+            for (int e = 0; e < E; ++e) x[e] = to_f32(k.v[e]);
+            fwht_wave<D>(x, lane);
+#pragma unroll
+            for (int e = 0; e < E; ++e) k.v[e] = store_rounded<IN>(x[e]);
+        }
+        reinterpret_cast<Lanes<IN, E>*>(tail)[lane] = k;
+        reinterpret_cast<Lanes<IN, E>*>(lds)[lane] = k;
+#pragma unroll
+        for (int e = 0; e < E; ++e) x[e] = to_f32(v.v[e]);
+        if constexpr (ROT) {
+            fwht_wave<D>(x, lane);
+#pragma unroll
+            for (int e = 0; e < E; ++e) x[e] = to_f32(store_rounded<IN>(x[e]));
+        }
+        float mn = x[0], mx = x[0];
+#pragma unroll
+        for (int e = 1; e < E; ++e) {
+            mn = __builtin_fminf(mn, x[e]);
+            mx = __builtin_fmaxf(mx, x[e]);
+        }
+        row_range<16>(mn, mx);
+        mn = -rows_max(-mn);
+        mx = rows_max(mx);
+        float s, b, inv;
+        qparams<BITS>(mn, mx, s, b, inv);
+        uint32_t w = 0;                                              // the lane's E codes, a byte each
+#pragma unroll
+        for (int e = 0; e < E; ++e)
+            w |= ((uint32_t)(int)qcode_f<BITS>(x[e], b, inv) & (BITS == 4 ? 0xFu : 0xFFu)) << (8 * e);
+        int bytes = E * lane;
+        bool mine = true;
+        if constexpr (BITS == 4) {                                   // dims D/2 on (lanes 32 on): the high nibbles
+            const auto o = __builtin_amdgcn_permlane32_swap(w, w, false, false);
+            w = o[0] | (o[1] << 4);
+            mine = lane < 32;
+        }
+        uint8_t* const codes = lds + D * sizeof(IN);
+        if (mine) {
+            const Lanes<uint8_t, E> c = __builtin_bit_cast(Lanes<uint8_t, E>, (std::conditional_t<E == 1, uint8_t, std::conditional_t<E == 2, uint16_t, uint32_t>>)w);
+            *reinterpret_cast<Lanes<uint8_t, E>*>(rec + F::OFF_VQ + slot * F::DC + bytes) = c;
+            *reinterpret_cast<Lanes<uint8_t, E>*>(codes + bytes) = c;
+        }
+        if (lane == 0) {
+            *reinterpret_cast<uint16_t*>(rec + F::OFF_VS + 2 * slot) = f16_bits(s);
+            *reinterpret_cast<uint16_t*>(rec + F::OFF_VB + 2 * slot) = f16_bits(b);
+            *reinterpret_cast<uint32_t*>(codes + F::DC) = (uint32_t)f16_bits(s) | ((uint32_t)f16_bits(b) << 16);
+        }
+    }
+    static constexpr int LDS = D * (int)sizeof(IN) + F::DC + 16;
+};
 
 // Split-K partials cross XCDs (separate L2s): stored write-through and read past the local L2, as
 // relaxed device-scope atomics (global_store / global_load with sc1).
@@ -894,7 +1068,7 @@ __device__ void merge_splits(const float* __restrict__ part_ml, const float* __r
 // (sequence, kv head, head chunk)), the last workgroup of a (sequence, kv head, head chunk) to
 // finish merges all splits into `out` and resets its counter, so no second launch is needed.
 template <int D, int BITS, typename IN, int NW, int ST, bool ROT, bool WS, int DEP>
-__global__ __launch_bounds__(NW * WAVE) __attribute__((amdgpu_waves_per_eu(2))) void decode_kernel(
+__global__ __launch_bounds__(NW * WAVE) __attribute__((amdgpu_waves_per_eu(2, D == 64 ? 4 : 2))) void decode_kernel(
     const IN* __restrict__ qg, IN* __restrict__ out, uint8_t* __restrict__ cache, int64_t bs, int64_t hs,
     IN* __restrict__ tail_k, const int32_t* __restrict__ tail_idx, const int32_t* __restrict__ block_table,
     const int32_t* __restrict__ seq_lens, int64_t bt_stride, int bt_cols, int H, int G, float p2, float rs, int NS,
@@ -927,6 +1101,7 @@ __global__ __launch_bounds__(NW * WAVE) __attribute__((amdgpu_waves_per_eu(2))) 
     __shared__ __align__(16) uint8_t ringB[2 * NW * R::SLOT];
     __shared__ __align__(16) uint8_t ringC[DEP == 3 ? 2 * NW * R::SLOT : 16];   // DEP = 3 only
     __shared__ __align__(16) int tbl[WIN];                               // block ids of the window
+    __shared__ __align__(16) uint8_t fresh[NewToken<D, BITS, IN>::LDS];   // the fused append's token (NewToken)
     float* const m_l = reinterpret_cast<float*>(ringB + AL::ML_OFF);      // after the loop only
     float* const l_l = m_l + NW * 16;
     int* const last_flag = reinterpret_cast<int*>(l_l + NW * 16);
@@ -970,22 +1145,35 @@ __global__ __launch_bounds__(NW * WAVE) __attribute__((amdgpu_waves_per_eu(2))) 
     const int hq = ST == 2 ? (r16 & 7) : r16;                            // the head of this lane's column
     const bool gv = hq < Gc;
     float qv[KSTEPS][8];
-    // ROT: the q rows in the butterfly layout instead (thread t: head t / QCG + QRP pp, dims 8 qc.. and
-    // D/2 + 8 qc..), rotated once the length is known
+    // RMF: a rotated cache's 16-bit q as loaded, rotated on the matrix cores (rotate_q). RLDS: an fp32 q in the
+    // butterfly layout instead (thread t: head t / QCG + QRP pp, dims 8 qc.. and D/2 + 8 qc..), rotated through LDS
+    // once the length is known
+    constexpr bool RMF = ROT && sizeof(IN) == 2, RLDS = ROT && !RMF;
     constexpr int QCG = D / 16, QRP = NW * WAVE / QCG, QPASS = (16 + QRP - 1) / QRP;
     const int qc = (int)threadIdx.x % QCG;
-    float qrow[ROT ? QPASS : 1][16];
-    if constexpr (ROT) {
+    float qrow[RLDS ? QPASS : 1][16];
+    u4 qraw[KSTEPS];
+    const IN* const qhead = qg + qbase + (int64_t)min(hq, Gc - 1) * D;
+    if constexpr (RLDS) {
 #pragma unroll
         for (int pp = 0; pp < QPASS; ++pp) {
             const int rr = min((int)threadIdx.x / QCG + pp * QRP, Gc - 1);
             load8(qg + qbase + (int64_t)rr * D + 8 * qc, reinterpret_cast<float(&)[8]>(qrow[pp][0]));
             load8(qg + qbase + (int64_t)rr * D + D / 2 + 8 * qc, reinterpret_cast<float(&)[8]>(qrow[pp][8]));
         }
+    } else if constexpr (RMF) {
+#pragma unroll
+        for (int kk = 0; kk < KSTEPS; ++kk) qraw[kk] = *reinterpret_cast<const u4*>(qhead + kdim<D, BITS>(kk, q, 0));
     } else {
 #pragma unroll
-        for (int kk = 0; kk < KSTEPS; ++kk) load8(qg + qbase + (int64_t)min(hq, Gc - 1) * D + kdim<D, BITS>(kk, q, 0), qv[kk]);
+        for (int kk = 0; kk < KSTEPS; ++kk) load8(qhead + kdim<D, BITS>(kk, q, 0), qv[kk]);
     }
+    // the new token's rows, which do not depend on the length either, in the wave that will append them: one that
+    // does not take the partial page, of the workgroup that holds the last split
+    const int aw = ws ? 0 : NW - 1;
+    NewToken<D, BITS, IN> token;
+    if (app_k != nullptr && zg == NSG - 1 && w == aw)
+        token.load(app_k + (int64_t)s * app_ks + (int64_t)h * D, app_v + (int64_t)s * app_vs + (int64_t)h * D, lane);
     constexpr int PRE = WIN / (NW * WAVE);                               // prefetched ids per thread
     const int npre = !ws && z == 0 ? min(WIN, bt_cols) : 0;
     int pre[PRE];
@@ -1004,28 +1192,38 @@ __global__ __launch_bounds__(NW * WAVE) __attribute__((amdgpu_waves_per_eu(2))) 
     const uint8_t* head_base = cache + (int64_t)h * hs;
 
     // Fused append (app_k): the token at position n - 1 of sequence s, kv head h, is written by the one
-    // workgroup that reads its page -- the split holding the page when the token completes it, else
-    // the last split (which takes the partial page) -- of the first head chunk (the entry point takes
-    // at most 16 q heads per kv head). Its stores are complete and visible to its own page loads after
-    // the barrier; no other workgroup reads that page or the sequence's tail.
-    if (app_k != nullptr) {
-        if (gc == 0 && n > 0) {
-            const int pos = n - 1, slot = pos % PAGE, pg = pos / PAGE;
-            const int owner = slot == PAGE - 1 ? pg / max(pps, 1) : NS - 1;
+    // workgroup that reads its page, of the first head chunk (the entry point takes at most 16 q heads per kv
+    // head). A token that completes its page goes first: the split that holds the page quantizes it, and its stores
+    // are complete and visible to its own page loads after the barrier. Else (31 tokens of 32) the last split,
+    // which takes the partial page, appends it behind its first page loads (NewToken). No other workgroup reads
+    // that page or the sequence's tail. One sequence of 333 tokens, 8 kv heads, rotated:
+    // 11.6 -> 9.1 us with rotate_q and the wave-wide output rotation; 200 sequences of 100-200 tokens: 34.7 -> 29.4 us.
+    bool appends = false;                                          // this workgroup holds the new token of a partial page
+    if (app_k != nullptr && gc == 0 && n > 0) {
+        const int pos = n - 1, slot = pos % PAGE, pg = pos / PAGE;
+        if (slot == PAGE - 1) {
+            const int owner = pg / max(pps, 1);
             if (zg == (ws ? owner / (NW * KW) : owner)) {           // the whole workgroup
                 const IN* krow = app_k + (int64_t)s * app_ks + (int64_t)h * D;
                 IN* tail = tail_k + ((int64_t)tix * H + h) * PAGE * D;
                 uint8_t* rec = cache + (int64_t)bt[pg] * bs + (int64_t)h * hs;
                 stash_rows<D, IN, true, ROT, NW * WAVE>(tail + slot * D, krow, 0, 1, (int)threadIdx.x);
-                page_task<D, BITS, IN, true, NW * WAVE, ROT>(tail, krow, 0, PAGE - 1, slot == PAGE - 1,
+                page_task<D, BITS, IN, true, NW * WAVE, ROT>(tail, krow, 0, PAGE - 1, true,
                                                              app_v + (int64_t)s * app_vs + (int64_t)h * D, 0, slot,
                                                              slot + 1, rec, ringA);
             }
+            __syncthreads();
+        } else {
+            appends = zg == NSG - 1;
         }
-        __syncthreads();
     }
     const bool has_tail = tail_n > 0 && zg == NSG - 1;                 // the workgroup holds the last split
     const int tail_blk = has_tail ? bt[full] : 0;                      // in before the page loop starts
+    const auto append_token = [&]() {
+        if (appends && w == aw)
+            token.template store<ROT>(tail_k + (((int64_t)tix * H + h) * PAGE + tail_n - 1) * D,
+                                      cache + (int64_t)tail_blk * bs + (int64_t)h * hs, tail_n - 1, fresh, lane);
+    };
     uint8_t* const sl0 = ringA + 2 * w * R::SLOT;
     uint8_t* const sl1 = sl0 + R::SLOT;
     uint8_t* const sl2 = ringB + 2 * w * R::SLOT;
@@ -1057,9 +1255,29 @@ __global__ __launch_bounds__(NW * WAVE) __attribute__((amdgpu_waves_per_eu(2))) 
     constexpr int NKP = AL::NKP, DS = D / (4 * NKP);
     constexpr bool TPRE = 2 * Packed<IN, DS>::WORDS <= (NW == 2 ? 32 : 16);
     const int tt = 16 * (w & 1) + r16, kp = w >> 1;
-    const int sdim = kp * (D / NKP) + q * DS;                          // first dim of the lane's slices
-    const IN* const ktail = tail_k + (((int64_t)tix * H + h) * PAGE + min(tt, tail_n - 1)) * D + sdim;
+    const IN* const ktail = tail_k + (((int64_t)tix * H + h) * PAGE + min(tt, tail_n - 1)) * D;
     Packed<IN, DS> kpk, qpk;
+    // The lane's slices: entries kp DS .. + DS - 1 of its q registers' (K-step, j), dims kdim(kk, q, j), the K-steps
+    // in the order that makes neighbours' dims adjacent (int4: the even ones, then the odd)
+    constexpr int RUN = Packed<IN, DS>::R;
+    const auto kstep = [](int x) { return BITS == 4 ? (x < KSTEPS / 2 ? 2 * x : 2 * x - KSTEPS + 1) : x; };
+    const auto tail_k_slices = [&](const IN* row) {
+#pragma unroll
+        for (int u = 0; u < DS / RUN; ++u) {
+            const int x = kp * DS + u * RUN;
+            kpk.load_run(u, row + kdim<D, BITS>(kstep(x / 8), q, x % 8));
+        }
+    };
+    const auto tail_q_slices = [&]() {
+#pragma unroll
+        for (int e = 0; e < DS; ++e) {
+            uint32_t x = 0;                                            // (masks: the registers must not be indexed)
+#pragma unroll
+            for (int c = 0; c < NKP; ++c)
+                x |= __float_as_uint(qv[kstep((c * DS + e) / 8)][(c * DS + e) % 8]) & (kp == c ? ~0u : 0u);
+            qpk.set(e, __uint_as_float(x));
+        }
+    };
     bool tpre = false, tdma = false;                                   // slices loaded, page DMA issued
 
     // The split's pages go out in pairs (k: pages 2k, 2k + 1 of the window), over windows of WIN pages
@@ -1119,16 +1337,14 @@ __global__ __launch_bounds__(NW * WAVE) __attribute__((amdgpu_waves_per_eu(2))) 
         __syncthreads();
         KUSH_MARK(1);
         KUSH_ISSUE_PAIR(sl0, sl1, pa)
-        // the tail's slices between the first pair and the rest: the first step's wait (the later
-        // pairs outstanding) then completes exactly the first pair and the slices, as with ROT
-        if (!ROT && TPRE && has_tail) {
-            kpk.load(ktail);
-            qpk.load(qg + qbase + (int64_t)min(r16, Gc - 1) * D + sdim);
-            tpre = true;
-        }
-        if constexpr (!ROT) KUSH_ISSUE_PAIR(sl2, sl3, pb)
+        // the tail's K slices between the first pair and the rest: the first step's wait (the later
+        // pairs outstanding) then completes exactly the first pair and the slices
+        if (TPRE && has_tail) tail_k_slices(ktail);
+        append_token();
+        if constexpr (!RLDS) KUSH_ISSUE_PAIR(sl2, sl3, pb)
         if constexpr (DEP == 3) KUSH_ISSUE_PAIR(sl4, sl5, pc)
-        if constexpr (ROT) {                                             // rotate, round to IN, regather
+        if constexpr (RMF) rotate_q<D, IN>(qraw, qv, lane);
+        if constexpr (RLDS) {                                            // rotate, round to IN, regather
             float* const qst = reinterpret_cast<float*>(ringB);          // [16][D]
 #pragma unroll
             for (int pp = 0; pp < QPASS; ++pp) {
@@ -1147,12 +1363,10 @@ __global__ __launch_bounds__(NW * WAVE) __attribute__((amdgpu_waves_per_eu(2))) 
             for (int kk = 0; kk < KSTEPS; ++kk)
 #pragma unroll
                 for (int j = 0; j < 8; ++j) qv[kk][j] = qst[min(hq, Gc - 1) * D + kdim<D, BITS>(kk, q, 0) + j];
-            if (TPRE && has_tail) {
-                kpk.load(ktail);
-#pragma unroll
-                for (int e = 0; e < DS; ++e) qpk.set(e, qst[min(r16, Gc - 1) * D + sdim + e]);
-                tpre = true;
-            }
+        }
+        if (TPRE && has_tail) {
+            tail_q_slices();
+            tpre = true;
         }
         // q' = q p2 as fp16 (+ its low part for fp32 q): qh, ql for the bias MFMAs; qa, qla the Q'
         // sources, divided by 16 in the int4 K-steps of high nibbles
@@ -1171,12 +1385,10 @@ __global__ __launch_bounds__(NW * WAVE) __attribute__((amdgpu_waves_per_eu(2))) 
                 qla[kk][j] = hin ? (_Float16)((float)lo * 0.0625f) : lo;
             }
         const float sa = rs * TWO24;                             // x = sa s + kx
-        if constexpr (ROT) {
+        if constexpr (RLDS) {
             __syncthreads();                                     // every wave done with the staged q
             KUSH_ISSUE_PAIR(sl2, sl3, pb)
-        }
-
-        // One pair step: the pair has landed once at most the other pair's loads are outstanding;
+        }        // One pair step: the pair has landed once at most the other pair's loads are outstanding;
         // scores of both pages (the next pair's table read hides behind them), one softmax update,
         // PV of both; then, every read of the
         // two slots complete (lgkmcnt 0), they take the next pair. The second page of a window's odd
@@ -1193,7 +1405,7 @@ __global__ __launch_bounds__(NW * WAVE) __attribute__((amdgpu_waves_per_eu(2))) 
             pair_scores2<D, BITS, QLO>(SA, qa, qla, qh, ql, sv, kx, rs, lane);                     \
             if (2 * (P) + 1 >= wn && r16 >= 8) kx = -__builtin_inff();   /* page B masked */        \
             id2 = *reinterpret_cast<const int2*>(tb + min(2 * nx, TW - 2));                        \
-            consume2<D, BITS>(SA, R::SLOT, o, vacc, sv, sa, kx, m_run, l_run, vb_run, lane);       \
+            consume2<D, BITS, vpre<D, BITS, DEP, WS>()>(SA, R::SLOT, o, vacc, sv, sa, kx, m_run, l_run, vb_run, lane);       \
         } else {                                                                                   \
             const uint8_t* const sp[2] = {SA, SB};                                                 \
             float sv[2][8], kx[2];                                                                 \
@@ -1205,7 +1417,7 @@ __global__ __launch_bounds__(NW * WAVE) __attribute__((amdgpu_waves_per_eu(2))) 
             const float pbm = 2 * (P) + 1 >= wn ? -__builtin_inff() : 0.0f;                        \
             _Pragma("unroll") for (int jj = 0; jj < 8; ++jj) sv[1][jj] += pbm;                     \
             id2 = *reinterpret_cast<const int2*>(tb + min(2 * nx, TW - 2));                        \
-            consume_pages<D, BITS, 2>(sp, o, vacc, sv, sa, kx, m_run, l_run, vb_run, lane);        \
+            consume_pages<D, BITS, 2, vpre<D, BITS, DEP, WS>()>(sp, o, vacc, sv, sa, kx, m_run, l_run, vb_run, lane);        \
         }                                                                                          \
         __builtin_amdgcn_s_waitcnt(0xC07F);                    /* lgkmcnt(0): slot reads done */    \
         const bool tl = (FIRST) && w == tw && has_tail && !tdma && nx >= pairs && wb + TW >= p1;       \
@@ -1248,6 +1460,9 @@ __global__ __launch_bounds__(NW * WAVE) __attribute__((amdgpu_waves_per_eu(2))) 
         if (ws) __syncthreads();                                 // every wave's pages done: rings idle
 #undef KUSH_STEP
 #undef KUSH_ISSUE_PAIR
+    } else if (appends) {                                        // no full page: the copies in LDS, before their use
+        append_token();
+        __syncthreads();
     }
     KUSH_MARK(3);
 
@@ -1260,8 +1475,8 @@ __global__ __launch_bounds__(NW * WAVE) __attribute__((amdgpu_waves_per_eu(2))) 
         uint8_t* const tslot = ringA + 2 * tw * R::SLOT;                   // wave tw's slot 0
         if (w == tw && !tdma) issue_page<D, BITS>(tslot, true, tail_blk, head_base, bs, voff);
         if (!tpre) {                                                       // the slices now
-            kpk.load(ktail);
-            if constexpr (ROT) {                                           // rotated q rows, as in the prologue
+            tail_k_slices(ktail);
+            if constexpr (RLDS) {                                          // rotated q rows, as in the prologue
                 for (int rr = (int)threadIdx.x / QCG; rr < 16; rr += QRP) {  // a row's lanes iterate together
                     float x[16];
                     load8(qg + qbase + (int64_t)min(rr, Gc - 1) * D + 8 * qc, reinterpret_cast<float(&)[8]>(x[0]));
@@ -1276,11 +1491,24 @@ __global__ __launch_bounds__(NW * WAVE) __attribute__((amdgpu_waves_per_eu(2))) 
                 }
                 __syncthreads();
 #pragma unroll
-                for (int e = 0; e < DS; ++e) qpk.set(e, qs[min(r16, Gc - 1) * QS + sdim + e]);
+                for (int e = 0; e < DS; ++e) {
+                    const int x = kp * DS + e;
+                    qpk.set(e, qs[min(hq, Gc - 1) * QS + kdim<D, BITS>(kstep(x / 8), q, x % 8)]);
+                }
             } else {
-                qpk.load(qg + qbase + (int64_t)min(r16, Gc - 1) * D + sdim);
+                if constexpr (RMF) {
+#pragma unroll
+                    for (int kk = 0; kk < KSTEPS; ++kk)
+                        qraw[kk] = *reinterpret_cast<const u4*>(qhead + kdim<D, BITS>(kk, q, 0));
+                    rotate_q<D, IN>(qraw, qv, lane);
+                } else {
+#pragma unroll
+                    for (int kk = 0; kk < KSTEPS; ++kk) load8(qhead + kdim<D, BITS>(kk, q, 0), qv[kk]);
+                }
+                tail_q_slices();
             }
         }
+        if (appends && tt == tail_n - 1) tail_k_slices(reinterpret_cast<const IN*>(fresh));   // the new token's row
         f4 c = f4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int e = 0; e < DS; ++e) c = __builtin_amdgcn_mfma_f32_16x16x4f32(qpk.get(e) * sm_log2, kpk.get(e), c, 0, 0, 0);
@@ -1297,12 +1525,24 @@ __global__ __launch_bounds__(NW * WAVE) __attribute__((amdgpu_waves_per_eu(2))) 
                 x[0][jj] = ST == 2 && r16 >= 8 ? -__builtin_inff() : v;
             }
             KUSH_WAIT_VM(0);
+            if (appends) {                                       // the new token's V row in place of the staged one
+                const uint8_t* const codes = fresh + D * sizeof(IN);
+                if (lane < F::DC / 4)
+                    *reinterpret_cast<uint32_t*>(tslot + slot_chunk<D, BITS>(31 + tail_n, lane / 4) + 4 * (lane % 4)) =
+                        *reinterpret_cast<const uint32_t*>(codes + 4 * lane);
+                if (lane == 0) {
+                    const uint32_t sb = *reinterpret_cast<const uint32_t*>(codes + F::DC);
+                    *reinterpret_cast<uint16_t*>(tslot + F::OFF_VS + 2 * (tail_n - 1)) = (uint16_t)sb;
+                    *reinterpret_cast<uint16_t*>(tslot + F::OFF_VB + 2 * (tail_n - 1)) = (uint16_t)(sb >> 16);
+                }
+                asm volatile("" ::: "memory");
+            }
             if constexpr (ST == 2) {                             // stream 0 takes the page
-                consume2<D, BITS>(tslot, 0, o, vacc, x[0], 1.0f, 0.0f, m_run, l_run, vb_run, lane);
+                consume2<D, BITS, vpre<D, BITS, DEP, WS>()>(tslot, 0, o, vacc, x[0], 1.0f, 0.0f, m_run, l_run, vb_run, lane);
             } else {
                 const uint8_t* const sp[1] = {tslot};
                 const float b0[1] = {0.0f};
-                consume_pages<D, BITS, 1>(sp, o, vacc, x, 1.0f, b0, m_run, l_run, vb_run, lane);
+                consume_pages<D, BITS, 1, vpre<D, BITS, DEP, WS>()>(sp, o, vacc, x, 1.0f, b0, m_run, l_run, vb_run, lane);
             }
         }
     }

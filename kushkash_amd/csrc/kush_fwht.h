@@ -57,6 +57,37 @@ __device__ __forceinline__ void fwht_runs(float (&x)[16], int c) {
 #pragma unroll
     for (int i = 0; i < 16; ++i) x[i] = x[i] * sc;
 }
+
+// The same transform with a whole wave per row: lane l holds the D / 64 consecutive dims x[e] = dim l D / 64 + e
+// (the same bits: the stages and their order are the same). A row's chain is then ~40 instructions where
+// fwht_runs spends ~200 on its 16 values per lane: for the few rows of a decode, whose latency counts.
+template <int D>
+__device__ __forceinline__ void fwht_wave(float (&x)[D / 64], int lane) {
+    constexpr int E = D / 64;
+#pragma unroll
+    for (int h = 1; h < E; h <<= 1) {                 // strides 1 .. E/2: within a lane
+#pragma unroll
+        for (int i = 0; i < E; ++i) {
+            if (i & h) continue;
+            const float a = x[i], b = x[i + h];
+            x[i] = a + b;
+            x[i + h] = a - b;
+        }
+    }
+    butterfly_lanes<1>(x, lane);                      // strides E .. 8 E: lane bits 0-3
+    butterfly_lanes<2>(x, lane);
+    butterfly_lanes<4>(x, lane);
+    butterfly_lanes<8>(x, lane);
+    const float sc = fwht_scale<D>();
+#pragma unroll
+    for (int i = 0; i < E; ++i) {                     // strides 16 E, 32 E: lane bits 4 and 5
+        auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x[i]), __float_as_uint(x[i]), false, false);
+        float y = __uint_as_float(a[0]) + __uint_as_float(a[1] ^ ((lane & 16) ? 0x80000000u : 0u));
+        auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(y), __float_as_uint(y), false, false);
+        y = __uint_as_float(b[0]) + __uint_as_float(b[1] ^ ((lane & 32) ? 0x80000000u : 0u));
+        x[i] = y * sc;
+    }
+}
 #pragma clang fp contract(on)
 
 }  // namespace kush
