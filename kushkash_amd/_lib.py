@@ -77,10 +77,22 @@ def lib() -> ctypes.CDLL:
 def call(name: str, *args) -> None:
     """Run one entry point; -1 (unsupported shape) -> ValueError like the reference's CPU path
     (kushkash/_cpu.py:38-40), any other failure -> RuntimeError with the library's message."""
-    rc = getattr(lib(), name)(*args)
+    check(name, getattr(lib(), name)(*args))
+
+
+def check(name: str, rc: int) -> None:
+    """Raise the error of an entry point that returned rc."""
     if rc == 0:
         return
     msg = (lib().kush_last_error() or b"").decode(errors="replace")
     if rc == -1:
         raise ValueError(msg)
     raise RuntimeError(f"{name} failed ({rc}): {msg}")
+
+
+PLAIN_CALL = call                # what `call` is unless someone records or replaces the launches
+
+
+def address(name: str) -> int:
+    """An entry point's address, for callers that hold it in native code."""
+    return ctypes.cast(getattr(lib(), name), ctypes.c_void_p).value

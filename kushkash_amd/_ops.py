@@ -137,6 +137,15 @@ class Ops:
         # counters of the fused split-K merge: zero at rest (the last workgroup of each (sequence, kv
         # head) resets its own), so one buffer serves every call of this Ops on one stream at a time
         self._sync = torch.zeros(SYNC_SLOTS, dtype=torch.int32, device=self.device)
+        try:
+            from . import _fastcall
+        except ImportError:                                     # not built: every call checks its arguments in Python
+            _fastcall = None
+        self._fast = _fastcall
+        if _fastcall is not None:
+            self._config = _fastcall.make_config(
+                head_dim, bits, group, self._dt, idx, self._sync.data_ptr(),
+                *(_lib.address(n) for n in ("kush_decode_ex", "kush_append_decode", "kush_write_ex")))
 
     # ---------------------------------------------------------------- argument checks
     def _validating(self) -> bool:
@@ -146,6 +155,24 @@ class Ops:
 
     def _stream(self) -> int:
         return torch.cuda.current_stream(self.device).cuda_stream
+
+    def _native(self) -> bool:
+        """Whether the per-step calls go through csrc/kush_fastcall.cpp (the same checks and launch, ~16 us of
+        Python in ~2): not where index values are to be checked, nor where the library calls are recorded."""
+        return self.gpu and self._fast is not None and not self.validate and self._lib.call is self._lib.PLAIN_CALL
+
+    def _native_decode(self, k, v, q, out, cache, block_table, seq_lens, tail_idx, tail_k, scale, n_splits, work, waves,
+                       order, rot) -> bool:
+        """decode (k None) or append_decode natively; False: not taken, nothing was launched."""
+        if waves is None:
+            waves = self.waves(q.shape[0], tail_k.shape[1], n_splits)
+        rc = self._fast.decode(self._config, k, v, q, out, cache, block_table, seq_lens, tail_idx, tail_k, scale, n_splits,
+                               work, waves, order, rot, SYNC_SLOTS, torch._C._cuda_getCurrentRawStream(self.device.index))
+        if rc == 0:
+            return True
+        if rc != self._fast.NOT_TAKEN:
+            self._lib.check("kush_decode_ex" if k is None else "kush_append_decode", rc)
+        return False
 
     def _on_device(self, **ts: torch.Tensor) -> None:
         for name, t in ts.items():
@@ -238,6 +265,13 @@ class Ops:
         build it) and runs both modes as one launch (mode 2), whose tail handling relies on that; under
         KUSHKASH_AMD_VALIDATE the declaration is checked and a list that misses a touched page raises.
         rot: as in append (rows from the chunk are rotated)."""
+        if fused and self._native():
+            rc = self._fast.write(self._config, k, v, query_start_loc, seq_lens, tail_idx, job_seq, job_page, cache,
+                                  block_table, tail_k, rot, torch._C._cuda_getCurrentRawStream(self.device.index))
+            if rc == 0:
+                return
+            if rc != self._fast.NOT_TAKEN:
+                self._lib.check("kush_write_ex", rc)
         n_jobs, H = job_seq.numel(), k.shape[1]
         if n_jobs == 0:
             return
@@ -396,6 +430,9 @@ class Ops:
         one Ops must not run concurrently on different streams (they share the counters, as the
         reference's callers share `work`). rot: the cache was written with rot=True: q is rotated on
         load and the output rotated back inside the kernels (no reference counterpart)."""
+        if self._native() and self._native_decode(None, None, q, out, cache, block_table, seq_lens, tail_idx, tail_k, scale,
+                                                  n_splits, work, waves, order, rot):
+            return
         self._decode(q, out, cache, block_table, seq_lens, tail_idx, tail_k, scale, n_splits, work, waves, order, rot,
                      None, None)
 
@@ -408,6 +445,9 @@ class Ops:
         calls): row s of k / v is the token at position seq_lens[s] - 1, which seq_lens already counts
         (the serving engines' convention). The same bytes and outputs as the two calls. No reference
         counterpart."""
+        if self._native() and self._native_decode(k, v, q, out, cache, block_table, seq_lens, tail_idx, tail_k, scale,
+                                                  n_splits, work, waves, order, rot):
+            return
         S, H = q.shape[0], tail_k.shape[1]
         self._check_rows("k", k, H)
         self._check_rows("v", v, H)

@@ -33,6 +33,9 @@ FLOOR_SOURCE = "kush_floor.hip"
 CPU_LIB = PKG / "libkushcpu.so"
 CPU_SOURCE = "kush_cpu.cpp"
 CPU_FLAGS = ["-O3", "-std=c++17", "-fPIC", "-shared", "-fopenmp", "-ffp-contract=off"]
+# The native host side of the per-step calls (csrc/kush_fastcall.cpp, a Python extension over torch's headers)
+FAST_LIB = PKG / "_fastcall.so"
+FAST_SOURCE = "kush_fastcall.cpp"
 SOURCES = ("kush_capi.hip", "kush_write.hip", "kush_decode.hip", "kush_rotate.hip",
            "kush_unpack.hip", "kush_attend.hip", "kush_decode_inst.hip")
 # the decode kernel instantiations: one object per (input dtype, rot)
@@ -164,10 +167,22 @@ def cxx() -> str:
     raise RuntimeError("g++ not found (the CPU path's library is built with it)")
 
 
+def fastcall_command(out: Path) -> list[str]:
+    """The compiler call that builds FAST_SOURCE against the torch it will run with."""
+    import sysconfig
+
+    import torch
+    base = Path(torch.__file__).resolve().parent
+    return [cxx(), "-O2", "-std=c++17", "-fPIC", "-shared", f"-I{base / 'include'}",
+            f"-I{base / 'include/torch/csrc/api/include'}", f"-I{sysconfig.get_paths()['include']}",
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-o", str(out),
+            str(PKG / "csrc" / FAST_SOURCE), f"-L{base / 'lib'}", "-ltorch_python", "-ltorch_cpu", "-lc10"]
+
+
 def build(verbose: bool = False, jobs: int | None = None) -> Path:
     """Compile every HIP source for gfx950 into LIB, TIMELINE_LIB from the same objects with the
-    timeline unit instrumented, the measurement library FLOOR_LIB, and the CPU path's host library
-    CPU_LIB (always recompiles; objects in parallel, then the links); returns LIB."""
+    timeline unit instrumented, the measurement library FLOOR_LIB, the CPU path's host library
+    CPU_LIB and the native host calls FAST_LIB (always recompiles; objects in parallel, then the links); returns LIB."""
     todo = units() + [(FLOOR_SOURCE, {}), (TIMELINE_UNIT[0], dict(TIMELINE_UNIT[1], KUSH_TIMELINE=1))]
     jobs = jobs or max(1, min(len(todo), int(os.environ.get("MAX_JOBS", 0)) or os.cpu_count() or 1))
     compile_flags = [f for f in FLAGS if f != "-shared"]
@@ -180,9 +195,12 @@ def build(verbose: bool = False, jobs: int | None = None) -> Path:
                          "-c", str(PKG / "csrc" / src), "-o", obj])
         cpu_tmp = CPU_LIB.with_suffix(".so.tmp")
         cmds.append([cxx(), *CPU_FLAGS, f"-I{ROOT / 'include'}", "-o", str(cpu_tmp), str(PKG / "csrc" / CPU_SOURCE)])
+        fast_tmp = FAST_LIB.with_suffix(".so.tmp")
+        cmds.append(fastcall_command(fast_tmp))
         with ThreadPoolExecutor(jobs) as ex:
             list(ex.map(lambda c: _run(c, verbose), cmds))
         os.replace(cpu_tmp, CPU_LIB)
+        os.replace(fast_tmp, FAST_LIB)
         product = objs[:len(units())]
         swap = units().index(TIMELINE_UNIT)
         timeline = product[:swap] + objs[-1:] + product[swap + 1:]
