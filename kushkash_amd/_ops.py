@@ -386,17 +386,37 @@ class Ops:
 
     # ---------------------------------------------------------------- decode
     def splits(self, num_seqs: int, num_kv_heads: int, max_full_pages: int) -> int:
-        """Split-K factor for MI355X: a power of two, doubled while the grid holds fewer workgroups
-        than CUs (a decode workgroup holds a whole CU's page ring) and every split keeps >= 2 pages per
-        wave; at most 256. As in the reference (_ops.py:182-189) the grid stays small, so a work
-        buffer of CUs * G * (D + 2) floats per (sequence, kv head) pair always suffices."""
-        ns = 1
+        """Split-K factor for MI355X, at most 256: 1 where the (sequence, kv head) pairs fill the CUs by themselves,
+        else the number of splits whose workgroups fill them evenly. A 4-wave workgroup's page ring takes 16
+        records of LDS:
+          over half a CU's (int8 at D 128, D 256)  as many splits as keep every workgroup resident at once, with
+            >= 3 pages per wave and split: past that a second round starts behind a nearly full first one
+            (19 sequences x 2 kv heads of D 256, ~4,500 tokens: 6 splits 34.2 us, 8 splits 45).
+          less (two fit a CU)  the fewest splits, of >= 2 pages per wave, that leave no more than a fifth of the
+            last round of CUs idle (18 x 8 heads of 6,000 tokens: 3 splits 33.3 us; 2 splits, some CUs with
+            two workgroups and the rest with one, 40.7), else the fullest.
+        Past 16 q heads per kv head (two workgroups on each page) a power of two of these (4 x 2 heads of 4,000
+        tokens, 20 q heads: 7 splits 16.1 us, 8 splits 15.2, 13 splits 17.7).
+        The grid stays within two workgroups per CU, as in the reference (_ops.py:182-189), so a work buffer
+        of 2 CUs * G * (D + 2) floats always suffices."""
         if not self.gpu:                                         # the host decode takes no splits (1 on CPU)
-            return ns
-        while (ns < 256 and num_seqs * num_kv_heads * ns < self.sms
-               and max_full_pages // (2 * ns) >= 2 * DECODE_WAVES):
-            ns *= 2
-        return ns
+            return 1
+        units = num_seqs * num_kv_heads * -(-self.G // 16)       # workgroups of one split
+        if units >= self.sms or units == 0:
+            return 1
+        single = 16 * record_bytes(self.D, self.bits) + 4 * 1024 > 80 * 1024
+        most = min(256, self.sms // units if single else 2 * self.sms // units,
+                   max_full_pages // ((3 if single else 2) * DECODE_WAVES))
+        best, fill = 1, 0.0
+        for ns in range(1, most + 1):
+            if self.G > 16 and ns & (ns - 1):
+                continue
+            share = units * ns / (self.sms * -(-units * ns // self.sms))
+            if share >= 0.8 and not single:
+                return ns
+            if share > fill:
+                best, fill = ns, share
+        return best
 
     def waves(self, num_seqs: int, num_kv_heads: int, n_splits: int, max_pages: int | None = None) -> int:
         """Waves per decode workgroup (measured on MI355X): 4 for split counts of 8 and more that 4
