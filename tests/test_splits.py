@@ -26,3 +26,30 @@ def test_split_policy(D, bits, G):
                 assert ns == 1 or pairs * chunks * ns <= ops.sms
     assert ops.splits(0, 8, 100) == 1
     assert ops.splits(8, 8, 4096) == (4 if chunks == 1 else 2)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D,bits,G,waves", [(128, 4, 7, 4), (128, 8, 4, 2), (256, 4, 16, 4), (64, 8, 2, 4)])
+@pytest.mark.parametrize("ns", [3, 5, 6, 7, 13])
+def test_any_split_count(D, bits, G, waves, ns):
+    """A step's append and decode in any number of splits, splits without pages and the token's page in any of them:
+    records and tails equal, outputs as in one split within their roundings."""
+    import torch
+    from test_gpu_append_decode import _state
+    lens = [0, 31, 95, 96, 160, 700, 1311, 2559]                        # before the token
+    S, H, dev = len(lens), 2, "cuda"
+    ops = Ops(torch.device(dev), D, bits, G, torch.bfloat16)
+    g = torch.Generator().manual_seed(ns)
+    k, v, q = (torch.randn(S, h, D, generator=g).to(torch.bfloat16).to(dev) for h in (H, H, H * G))
+    sl = torch.tensor([n + 1 for n in lens], dtype=torch.int32, device=dev)
+    got = []
+    for n in (1, ns):
+        cache, bt, tail_k, tail_idx = _state(ops, lens, H, D, torch.bfloat16, seed=D + bits)
+        out, work = torch.empty_like(q), torch.empty(S * H * n * G * (D + 2), device=dev)
+        ops.append_decode(k, v, q, out, cache, bt, sl, tail_idx, tail_k, D ** -0.5, n, work, waves=waves)
+        got.append((cache, tail_k, out.float()))
+    (c1, t1, a), (c2, t2, b) = got
+    assert torch.equal(c1, c2) and torch.equal(t1, t2)
+    # a weight is rounded to fp16 once per launch, relative to another split's largest score (unit roundoff 2^-11, two
+    # launches, values' code part below 6), and each output once to bf16 (2^-8 of it, both)
+    assert ((a - b).abs() <= 2 * 2.0 ** -11 * 6 + 2.0 ** -7 * torch.maximum(a.abs(), b.abs())).all()
