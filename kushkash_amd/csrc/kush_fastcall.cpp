@@ -4,7 +4,9 @@
 //
 // Each function returns the library's code, or NOT_TAKEN for anything that is not the plain, valid case -- a
 // tensor subclass or one without storage, a wrong type, shape, stride, device or alignment, an option it does not
-// know. The caller then takes its Python path, which makes the same checks and raises the errors.
+// know. The caller then takes its Python path, which makes the same checks and raises the errors. Every pointer is
+// read before the GIL is released: data_ptr() throws for a tensor without storage (what torch.vmap passes is of
+// type torch.Tensor too), and a thrown exception must find the thread state in place.
 #include <Python.h>
 #include <torch/csrc/autograd/python_variable.h>
 
@@ -61,25 +63,31 @@ const at::Tensor* rows(const Config& c, PyObject* o, int64_t H) {
                : nullptr;
 }
 
-uint64_t addr(const at::Tensor& t) { return (uint64_t)(uintptr_t)t.data_ptr(); }
 template <typename T>
 T* ptr(const at::Tensor& t) { return static_cast<T*>(t.data_ptr()); }
 
-// The paged cache of H kv heads
+// The paged cache of H kv heads; block_table of `seqs` rows, `cols` pages each
 struct Cache {
-    const at::Tensor *cache, *table, *tail;
-    int64_t bs, hs;
+    void *cache, *tail;
+    const int32_t* table;
+    int64_t bs, hs, H, seqs, cols, row;
     bool take(const Config& c, PyObject* oc, PyObject* ot, PyObject* ok) {
-        cache = tensor(c, oc);
-        table = tensor(c, ot);
-        tail = tensor(c, ok);
-        if (!cache || !table || !tail || tail->dim() != 4 || cache->dim() < 2) return false;
-        const int64_t H = tail->size(1), e = cache->element_size();
-        bs = cache->stride(0) * e;
-        hs = cache->stride(1) * e;
-        return cache->size(1) >= H && ((addr(*cache) | (uint64_t)bs | (uint64_t)hs) & 15) == 0 && tail->size(2) == PAGE &&
-               tail->size(3) == c.D && tail->is_contiguous() && tail->scalar_type() == c.type && table->dim() == 2 &&
-               table->scalar_type() == at::kInt && table->stride(1) == 1;
+        const at::Tensor *tc = tensor(c, oc), *tt = tensor(c, ot), *tk = tensor(c, ok);
+        if (!tc || !tt || !tk || tk->dim() != 4 || tc->dim() < 2 || tt->dim() != 2) return false;
+        const int64_t e = tc->element_size();
+        H = tk->size(1);
+        bs = tc->stride(0) * e;
+        hs = tc->stride(1) * e;
+        seqs = tt->size(0);
+        cols = tt->size(1);
+        row = tt->stride(0);
+        if (tc->size(1) < H || tk->size(2) != PAGE || tk->size(3) != c.D || !tk->is_contiguous() ||
+            tk->scalar_type() != c.type || tt->scalar_type() != at::kInt || tt->stride(1) != 1)
+            return false;
+        cache = tc->data_ptr();
+        tail = tk->data_ptr();
+        table = ptr<int32_t>(*tt);
+        return (((uint64_t)(uintptr_t)cache | (uint64_t)bs | (uint64_t)hs) & 15) == 0;
     }
 };
 
@@ -102,13 +110,13 @@ long decode(PyObject* const* a) {
         !integer(a[17], stream) || !PyBool_Check(a[15]) || !PyFloat_CheckExact(a[10]))
         return NOT_TAKEN;
     const at::Tensor *q = tensor(c, a[3]), *out = tensor(c, a[4]);
-    const int64_t H = s.tail->size(1);
+    const int64_t H = s.H;
     if (!q || !out || q->dim() != 3 || q->size(1) != H * c.G || q->size(2) != c.D || !q->is_contiguous() ||
         q->scalar_type() != c.type || out->sizes() != q->sizes() || !out->is_contiguous() || out->scalar_type() != c.type)
         return NOT_TAKEN;
     const int64_t S = q->size(0), rows_ = S * H * ns * c.G;
     const at::Tensor *lens = index32(c, a[7], S), *tidx = index32(c, a[8], S);
-    if (!lens || !tidx || s.table->size(0) < S || ns < 1 || ns > (1 << 20) || waves < 0 || waves > 8 || S > INT32_MAX ||
+    if (!lens || !tidx || s.seqs < S || ns < 1 || ns > (1 << 20) || waves < 0 || waves > 8 || S > INT32_MAX ||
         H > INT32_MAX)
         return NOT_TAKEN;
     float *ml = nullptr, *po = nullptr;
@@ -122,30 +130,32 @@ long decode(PyObject* const* a) {
     }
     const at::Tensor* order = a[14] == Py_None ? nullptr : index32(c, a[14], S);
     if (a[14] != Py_None && !order) return NOT_TAKEN;
-    const int32_t cols = (int32_t)std::min<int64_t>(s.table->size(1), 1 << 30);
+    const int32_t cols = (int32_t)std::min<int64_t>(s.cols, 1 << 30);
     int32_t* const sync = ns > 1 ? c.sync : nullptr;
     const int32_t* const ord = order ? ptr<int32_t>(*order) : nullptr;
     const float scale = (float)PyFloat_AS_DOUBLE(a[10]);
     const int rot = a[15] == Py_True;
+    const void* const pq = q->data_ptr();
+    void* const pout = out->data_ptr();
+    const int32_t *const ptidx = ptr<int32_t>(*tidx), *const plens = ptr<int32_t>(*lens);
     if (a[1] == Py_None) {
         int rc;
         Py_BEGIN_ALLOW_THREADS;
-        rc = c.decode(c.D, c.bits, c.G, c.dtype, q->data_ptr(), out->data_ptr(), s.cache->data_ptr(), s.bs, s.hs,
-                      s.tail->data_ptr(), ptr<int32_t>(*tidx), ptr<int32_t>(*s.table), ptr<int32_t>(*lens),
-                      s.table->stride(0), H, scale, ns, ml, po, S, (void*)stream, cols, sync, waves, ord, rot);
+        rc = c.decode(c.D, c.bits, c.G, c.dtype, pq, pout, s.cache, s.bs, s.hs, s.tail, ptidx, s.table, plens, s.row, H,
+                      scale, ns, ml, po, S, (void*)stream, cols, sync, waves, ord, rot);
         Py_END_ALLOW_THREADS;
         return rc;
     }
     const at::Tensor *k = rows(c, a[1], H), *v = rows(c, a[2], H);
     if (!k || !v || k->size(0) < S || v->size(0) < S || c.G > 16) return NOT_TAKEN;
     const uint64_t e = k->element_size();
-    if ((addr(*k) | addr(*v) | k->stride(0) * e | v->stride(0) * e) & 15) return NOT_TAKEN;
+    const void *const pk = k->data_ptr(), *const pv = v->data_ptr();
+    const int64_t ks = k->stride(0), vs = v->stride(0);
+    if (((uint64_t)(uintptr_t)pk | (uint64_t)(uintptr_t)pv | ks * e | vs * e) & 15) return NOT_TAKEN;
     int rc;
     Py_BEGIN_ALLOW_THREADS;
-    rc = c.append_decode(c.D, c.bits, c.G, c.dtype, q->data_ptr(), out->data_ptr(), s.cache->data_ptr(), s.bs, s.hs,
-                         s.tail->data_ptr(), ptr<int32_t>(*tidx), ptr<int32_t>(*s.table), ptr<int32_t>(*lens),
-                         s.table->stride(0), H, scale, ns, ml, po, S, (void*)stream, k->data_ptr(), v->data_ptr(),
-                         k->stride(0), v->stride(0), cols, sync, waves, ord, rot);
+    rc = c.append_decode(c.D, c.bits, c.G, c.dtype, pq, pout, s.cache, s.bs, s.hs, s.tail, ptidx, s.table, plens, s.row, H,
+                         scale, ns, ml, po, S, (void*)stream, pk, pv, ks, vs, cols, sync, waves, ord, rot);
     Py_END_ALLOW_THREADS;
     return rc;
 }
@@ -160,22 +170,25 @@ long write(PyObject* const* a) {
     if (!k || k->dim() != 3 || !integer(a[12], stream) || !PyBool_Check(a[11])) return NOT_TAKEN;
     const int64_t H = k->size(1);
     const at::Tensor* v = rows(c, a[2], H);
-    if (!rows(c, a[1], H) || !v || !s.take(c, a[8], a[9], a[10]) || s.tail->size(1) != H) return NOT_TAKEN;
+    if (!rows(c, a[1], H) || !v || !s.take(c, a[8], a[9], a[10]) || s.H != H) return NOT_TAKEN;
     const at::Tensor *qsl = index32(c, a[3], 0), *lens = index32(c, a[4], 0), *tidx = index32(c, a[5], 0),
                      *js = index32(c, a[6], 1), *jp = index32(c, a[7], 1);
     if (!qsl || !lens || !tidx || !js || !jp || js->numel() != jp->numel() || js->numel() > INT32_MAX || H > INT32_MAX)
         return NOT_TAKEN;
+    const void *const pk = k->data_ptr(), *const pv = v->data_ptr();
+    const int32_t *const pqsl = ptr<int32_t>(*qsl), *const plens = ptr<int32_t>(*lens), *const ptidx = ptr<int32_t>(*tidx),
+                  *const pjs = ptr<int32_t>(*js), *const pjp = ptr<int32_t>(*jp);
+    const int64_t ks = k->stride(0), vs = v->stride(0), jobs = js->numel();
+    const int rot = a[11] == Py_True;
     int rc;
     Py_BEGIN_ALLOW_THREADS;
-    rc = c.write(c.D, c.bits, c.dtype, k->data_ptr(), v->data_ptr(), k->stride(0), v->stride(0), ptr<int32_t>(*qsl),
-                 ptr<int32_t>(*lens), ptr<int32_t>(*tidx), ptr<int32_t>(*js), ptr<int32_t>(*jp), js->numel(), 2,
-                 s.cache->data_ptr(), s.bs, s.hs, s.tail->data_ptr(), ptr<int32_t>(*s.table), s.table->stride(0), H,
-                 (void*)stream, a[11] == Py_True);
+    rc = c.write(c.D, c.bits, c.dtype, pk, pv, ks, vs, pqsl, plens, ptidx, pjs, pjp, jobs, 2, s.cache, s.bs, s.hs, s.tail,
+                 s.table, s.row, H, (void*)stream, rot);
     Py_END_ALLOW_THREADS;
     return rc;
 }
 
-// A tensor without storage throws on its pointer: not taken either
+// A tensor without storage throws on its pointer, with the GIL held: not taken either
 template <long (*F)(PyObject* const*), int N>
 PyObject* entry(PyObject*, PyObject* const* args, Py_ssize_t n) {
     long rc = NOT_TAKEN;

@@ -81,3 +81,16 @@ def test_the_same_errors(what):
             ops.append_decode(**a)
         said.append((type(e.value), str(e.value)))
     assert said[0] == said[1]
+
+
+@pytest.mark.parametrize("name", ["q", "seq_lens"])
+def test_a_tensor_without_storage(name):
+    """What torch.vmap passes is a torch.Tensor by type: refused as on the Python path, before any launch."""
+    said = []
+    for native in (True, False):
+        ops = _ops(native)
+        a = _step(ops, 1)
+        with pytest.raises(RuntimeError) as e:
+            torch.vmap(lambda x: ops.append_decode(**{**a, name: x}))(a[name][None])
+        said.append(str(e.value))
+    assert said[0] == said[1]
