@@ -37,8 +37,9 @@ def _plain(*ts: torch.Tensor) -> bool:
         return False
     if torch.is_grad_enabled() and any(t.requires_grad for t in ts):
         return False
-    return not (torch.compiler.is_compiling() or torch._C._functorch.peek_interpreter_stack() is not None
-                or torch._C._len_torch_dispatch_stack() or torch.autograd.forward_ad._current_level >= 0)
+    return not (torch.compiler.is_compiling() or torch._C._get_tracing_state() is not None      # (torch.jit.trace)
+                or torch._C._functorch.peek_interpreter_stack() is not None or torch._C._len_torch_dispatch_stack()
+                or torch.autograd.forward_ad._current_level >= 0)
 
 
 def _row_strides(t: torch.Tensor, D: int) -> tuple[int, int, int]:

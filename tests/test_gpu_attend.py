@@ -94,6 +94,25 @@ def test_inputs_left_to_the_other_paths():
         assert _attend.takes(q, k, v, 0.1)
 
 
+def test_a_trace_is_not_plain():
+    """torch.jit.trace records torch's operators only: under it nothing is the kernel's."""
+    x, seen = torch.randn(2, 4), []
+    torch.jit.trace(lambda t: seen.append(_attend._plain(t)) or t + 1, x, check_trace=False)
+    assert seen == [False] and _attend._plain(x)
+
+
+@pytest.mark.gpu
+def test_a_traced_prompt_attends_its_own_inputs():
+    """(One q head per kv head: torch cannot trace repeat_interleave, which the path left to torch needs for more.)"""
+    from kushkash_amd.hf import prompt_attention
+    torch.manual_seed(7)
+    first, second = ([torch.randn(1, h, 70, 128, device=DEV).bfloat16() for h in (2, 2, 2)] for _ in range(2))
+    traced = torch.jit.trace(lambda q, k, v: prompt_attention(q, k, v, 0.09), first, check_trace=False)
+    for x in (first, second):
+        want = _exact(*(t[0].transpose(0, 1) for t in x), True, 0.09)[0].transpose(0, 1)
+        assert _rel(traced(*x)[0], want) < BOUND[torch.bfloat16]
+
+
 @pytest.mark.parametrize("G", [1, 4, 7, 16])
 def test_the_plan_covers_the_keys_and_bounds_its_scratch(G):
     """Whatever the shape: 4 or 8 waves, a split (if any) of at least 12 key tiles that leaves more than one
