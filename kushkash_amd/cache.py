@@ -222,8 +222,10 @@ class KushCache:
         # rows it stores are rotated by the product (the rotations agree to fp32 rounding, and the output is
         # rounded once instead of twice): one launch for the nine of q's and the output's conversions,
         # products and scalings around it (4 sequences of 1,000 tokens, fp16: 96 -> 19 us a pass). The launch would
-        # rotate a token's rows too, so product-rotated ones are appended by a launch of their own.
-        rot = self.rot is not None and self.gpu
+        # rotate a token's rows too, so product-rotated ones are appended by a launch of their own. A q that the
+        # cache's dtype does not hold is rotated by the product, from its own values: the launch would round it twice.
+        held = q.dtype == self.kdtype or self.kdtype == torch.float32
+        rot = self.krot or (self.rot is not None and self.gpu and held)
         qk = (q.to(self.kdtype) if rot else self._inward(q)).contiguous()
         out = torch.empty_like(qk)
         pages = (self._capacity if self._splits else self._tokens[layer]) // PAGE

@@ -163,3 +163,35 @@ def test_attend_chunk_memory_is_bounded():
     assert extra <= 1 << 30, f"attend_chunk took {extra / 2**20:.0f} MiB beyond the cache"
     ref = history_attention(q, k, v, c.pool[0], c.block_table, N, c.tail_k[0], D, 4, c.scale)
     assert_out_close(out, ref.float(), torch.bfloat16, base=1e-3, roundings=2, what="attend_chunk vs the torch path")
+
+
+@pytest.mark.parametrize("cache_dtype,q_dtype", [(torch.bfloat16, torch.float32), (torch.float16, torch.float32),
+                                                 (torch.float16, torch.bfloat16), (torch.float32, torch.bfloat16),
+                                                 (torch.bfloat16, torch.bfloat16)])
+@pytest.mark.parametrize("append", [False, True])
+def test_q_of_another_dtype_is_rounded_once(cache_dtype, q_dtype, append):
+    """A product-rotated cache's q, whatever its dtype: rotated from the values given and rounded once to the cache's
+    dtype. Where the cache's dtype does not hold q, that is the rotation by the product around an unrotated launch, bit
+    for bit; where it does, the launch rotates q (the same value but for the order of its fp32 sums)."""
+    from kushkash_amd._rotation import rotate
+    B, Hq, Hkv, D, n = 2, 8, 2, 128, 75
+    g = torch.Generator().manual_seed(5)
+    c = kk.KushCache(1, Hkv, Hq, D, batch_size=B, bits=4, device=DEV, dtype=cache_dtype, rotate=True)
+    rows = [torch.randn(B, Hkv, n + 1, D, generator=g).to(cache_dtype).to(DEV) for _ in range(2)]
+    c.write(0, *(x[:, :, :n] for x in rows))
+    q = (torch.randn(B, Hq, D, generator=g) * 3).to(q_dtype).to(DEV)
+    out = c.append_attend(0, q, *(x[:, :, n:] for x in rows)) if append else c.attend(0, q)
+    seen = []
+    real, c.ops.decode = c.ops.decode, lambda *a, **kw: seen.append(kw.get("rot", False)) or real(*a, **kw)
+    again = c.attend(0, q)
+    assert torch.equal(again, out) and out.dtype == cache_dtype
+    exact = cache_dtype in (q_dtype, torch.float32)
+    assert seen == [exact]
+    want = torch.empty(B, Hq, D, dtype=cache_dtype, device=DEV)
+    real(rotate(q, c.rot, cache_dtype), want, c.pool[0], c.block_table, c.seq_lens[0], c.tail_idx, c.tail_k[0], c.scale)
+    want = rotate(want, c.rot)
+    if exact:
+        # an fp32 sum's last bit may flip one rounding of a q dim, and the product's way rounds its output twice
+        assert ((out - want).norm() / want.norm()).item() < 4 * torch.finfo(cache_dtype).eps
+    else:
+        assert torch.equal(out, want)
