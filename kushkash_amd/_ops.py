@@ -24,6 +24,7 @@ from __future__ import annotations
 import math
 import os
 from dataclasses import dataclass
+from functools import lru_cache
 
 import torch
 
@@ -94,6 +95,45 @@ def check_unpack_indices(page_blk: torch.Tensor, page_dst: torch.Tensor, tail_bl
     if bad:
         raise ValueError(f"unpack: index out of range: {', '.join(bad)} "
                          f"({rows} rows, {blocks} blocks, {slots} tail slots, 1..{PAGE} tokens per partial page)")
+
+
+@lru_cache(4096)
+def _split_count(sms: int, units: int, pages: int, record: int, chunked: bool) -> int:
+    """Splits of a decode whose unsplit grid is `units` workgroups over at most `pages` full pages each. A 4-wave
+    workgroup's page ring takes 16 records of LDS: over half a CU's (int8 at D 128, D 256) every workgroup is to be
+    resident at once (past that a second round starts behind a nearly full first one: 19 sequences x 2 kv heads of
+    D 256, ~4,500 tokens: 6 splits 34.2 us, 8 splits 45), else two or more share a CU. Every split keeps 2 pages
+    per wave. Of these counts, the least estimate in steps of a page pair:
+      the pairs of one wave, halfway between their mean and the busiest wave's whole number of them, each twice as
+        long where CUs hold two workgroups (1.8 times where three fit: D 64, int4);
+      + (2 + 0.2 splits) sqrt(4736 / record) for the merge, whose time grows less than the pages' with the record.
+    The constants are the best of a grid of them over 542 measured points (ten record formats and head groups, 1-14
+    sequences, 300-65,536 tokens, up to 35 counts each): 3.3 % over each point's fastest count on average. Powers of
+    two until the grid holds as many workgroups as CUs were 13 % over; the first count that leaves at most a fifth of
+    the CUs idle 6 %, and up to 10 % behind the powers of two where those fill the CUs exactly (int4, 8 kv heads,
+    4 sequences of 4,096 tokens: 7 splits 14.3 us, 8 splits 13.7; 2 of 131,072: 13 splits 69.9 us, 16 splits 66.6).
+    The most that this rule is behind either is 4.4 %.
+    Two at least where they fit: a row's weights are rounded to fp16 relative to the largest of their split and wave,
+    so fewer splits are less exact (1,000 tokens, fp16: 2.90e-4 from 64 bits at 1 split, 2.71e-4 at 3, 2.62e-4 at 8),
+    and one split would save ~1 us of 12 up to 1,000 tokens.
+    chunked: past 16 q heads per kv head (two workgroups on each page) powers of two alone (4 x 2 heads of 4,000
+    tokens, 20 q heads: 7 splits 16.1 us, 8 splits 15.2, 13 splits 17.7)."""
+    if units >= sms or units == 0:
+        return 1
+    single = 16 * record + 4 * 1024 > 80 * 1024
+    shared = 1.8 if 16 * record + 4 * 1024 <= 54 * 1024 else 2.0
+    merge = math.sqrt(4736 / record)
+    most = min(256, (sms if single else 2 * sms) // units, pages // (2 * DECODE_WAVES))
+    best, least = 1, math.inf
+    for ns in range(2 if most >= 2 and 2 * units <= sms else 1, most + 1):
+        if chunked and ns & (ns - 1):
+            continue
+        pairs = -(-(-(-pages // ns)) // 2)
+        steps = (-(-pairs // DECODE_WAVES) + pairs / DECODE_WAVES) / 2
+        cost = steps * (1.0 if units * ns <= sms else shared) + ((2 + 0.2 * ns) * merge if ns > 1 else 0.0)
+        if cost < least:
+            best, least = ns, cost
+    return best
 
 
 class Ops:
@@ -387,36 +427,12 @@ class Ops:
     # ---------------------------------------------------------------- decode
     def splits(self, num_seqs: int, num_kv_heads: int, max_full_pages: int) -> int:
         """Split-K factor for MI355X, at most 256: 1 where the (sequence, kv head) pairs fill the CUs by themselves,
-        else the number of splits whose workgroups fill them evenly. A 4-wave workgroup's page ring takes 16
-        records of LDS:
-          over half a CU's (int8 at D 128, D 256)  as many splits as keep every workgroup resident at once, with
-            >= 3 pages per wave and split: past that a second round starts behind a nearly full first one
-            (19 sequences x 2 kv heads of D 256, ~4,500 tokens: 6 splits 34.2 us, 8 splits 45).
-          less (two fit a CU)  the fewest splits, of >= 2 pages per wave, that leave no more than a fifth of the
-            last round of CUs idle (18 x 8 heads of 6,000 tokens: 3 splits 33.3 us; 2 splits, some CUs with
-            two workgroups and the rest with one, 40.7), else the fullest.
-        Past 16 q heads per kv head (two workgroups on each page) a power of two of these (4 x 2 heads of 4,000
-        tokens, 20 q heads: 7 splits 16.1 us, 8 splits 15.2, 13 splits 17.7).
-        The grid stays within two workgroups per CU, as in the reference (_ops.py:182-189), so a work buffer
-        of 2 CUs * G * (D + 2) floats always suffices."""
+        else the count that _split_count estimates to be the fastest. The grid stays within two workgroups per
+        CU, as in the reference (_ops.py:182-189), so a work buffer of 2 CUs * G * (D + 2) floats always suffices."""
         if not self.gpu:                                         # the host decode takes no splits (1 on CPU)
             return 1
-        units = num_seqs * num_kv_heads * -(-self.G // 16)       # workgroups of one split
-        if units >= self.sms or units == 0:
-            return 1
-        single = 16 * record_bytes(self.D, self.bits) + 4 * 1024 > 80 * 1024
-        most = min(256, self.sms // units if single else 2 * self.sms // units,
-                   max_full_pages // ((3 if single else 2) * DECODE_WAVES))
-        best, fill = 1, 0.0
-        for ns in range(1, most + 1):
-            if self.G > 16 and ns & (ns - 1):
-                continue
-            share = units * ns / (self.sms * -(-units * ns // self.sms))
-            if share >= 0.8 and not single:
-                return ns
-            if share > fill:
-                best, fill = ns, share
-        return best
+        return _split_count(self.sms, num_seqs * num_kv_heads * -(-self.G // 16), max_full_pages,
+                            record_bytes(self.D, self.bits), self.G > 16)
 
     def waves(self, num_seqs: int, num_kv_heads: int, n_splits: int, max_pages: int | None = None) -> int:
         """Waves per decode workgroup (measured on MI355X): 4 for split counts of 8 and more that 4

@@ -28,6 +28,17 @@ def test_split_policy(D, bits, G):
     assert ops.splits(8, 8, 4096) == (4 if chunks == 1 else 2)
 
 
+# sequences, kv heads, D, bits, tokens and the counts within a few percent of the fastest one, as measured
+@pytest.mark.parametrize("S,H,D,bits,tokens,good", [
+    (12, 4, 128, 4, 1000, (2, 3)), (4, 8, 128, 4, 4096, (8,)), (2, 8, 128, 4, 131072, (16,)),
+    (1, 8, 128, 4, 131072, (26, 32)), (8, 8, 128, 4, 131072, (3, 4)), (3, 8, 64, 4, 32768, (10, 21)),
+    (2, 8, 64, 4, 65536, (16,)), (1, 4, 256, 8, 4096, (8, 16))])
+def test_small_batches_fill_the_chip(S, H, D, bits, tokens, good):
+    ops = Ops.__new__(Ops)
+    ops.D, ops.bits, ops.G, ops.gpu, ops.sms = D, bits, 4, True, 256
+    assert ops.splits(S, H, tokens // 32) in good
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("D,bits,G,waves", [(128, 4, 7, 4), (128, 8, 4, 2), (256, 4, 16, 4), (64, 8, 2, 4)])
 @pytest.mark.parametrize("ns", [3, 5, 6, 7, 13])
