@@ -142,7 +142,7 @@ def prompt_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: f
     illegal-address fault on this device. torch's half-precision math path (batched products over
     transposed views) is never taken either."""
     rows = [x.transpose(1, 2) for x in (q, k, v)]
-    if _attend.takes(*rows, scale):
+    if k.shape[2] == q.shape[2] and _attend.takes(*rows, scale):     # else query t sees keys 0 .. t all the same
         return _attend.attend(*rows, True, scale).transpose(1, 2)
     if q.dtype in (torch.float16, torch.bfloat16):
         g = q.shape[1] // k.shape[1]

@@ -113,6 +113,23 @@ def test_a_traced_prompt_attends_its_own_inputs():
         assert _rel(traced(*x)[0], want) < BOUND[torch.bfloat16]
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("N", [40, 64, 100, 150])
+def test_a_prompt_over_keys_of_another_length(N):
+    """prompt_attention with more or fewer keys than queries: query t sees keys 0 .. t, as the paths around the kernel
+    have it (the kernel aligns the queries with the last keys, and takes no causal call of fewer keys than queries)."""
+    from kushkash_amd.hf import prompt_attention
+    torch.manual_seed(N)
+    T, scale = 100, 0.09
+    q, k, v = (torch.randn(1, h, n, 128, device=DEV).bfloat16() for h, n in ((4, T), (2, N), (2, N)))
+    got = prompt_attention(q, k, v, scale)
+    s = torch.stack([q[0, h].double().cpu() @ k[0, h // 2].double().cpu().t() for h in range(4)]) * scale
+    s.masked_fill_(torch.arange(N) > torch.arange(T)[:, None], -math.inf)
+    p = torch.softmax(s, -1)
+    want = torch.stack([p[h] @ v[0, h // 2].double().cpu() for h in range(4)])
+    assert got.dtype == q.dtype and _rel(got[0], want) < BOUND[torch.bfloat16]
+
+
 @pytest.mark.parametrize("G", [1, 4, 7, 16])
 def test_the_plan_covers_the_keys_and_bounds_its_scratch(G):
     """Whatever the shape: 4 or 8 waves, a split (if any) of at least 12 key tiles that leaves more than one
