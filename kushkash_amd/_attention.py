@@ -235,7 +235,11 @@ def _unpacked_rows(ops, k_new: torch.Tensor, v_new: torch.Tensor, cache: torch.T
             return r
         return (torch.arange(0, B * rows, rows, device=dev, dtype=torch.int32)[:, None] + r).view(-1)
 
-    new = [x.transpose(1, 2).reshape(B * T, Hk, D) for x in (k_new, v_new)]
+    def rows_of(x: torch.Tensor) -> torch.Tensor:                          # the unpack's rows: heads D apart
+        y = x.transpose(1, 2).reshape(B * T, Hk, D)                        # (B = 1: a view, of any strides)
+        return y if y.stride(2) == 1 and y.stride(1) == D else y.reshape(-1).view(B * T, Hk, D)
+
+    new = [rows_of(x) for x in (k_new, v_new)]
     kp, vp = (torch.empty(B, rows, Hk, D, dtype=ops.dtype, device=dev) for _ in range(2))
     tail_blk = info = torch.zeros(0, dtype=torch.int32, device=dev)
     if n_hist % PAGE:

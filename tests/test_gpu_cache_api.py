@@ -195,3 +195,20 @@ def test_q_of_another_dtype_is_rounded_once(cache_dtype, q_dtype, append):
         assert ((out - want).norm() / want.norm()).item() < 4 * torch.finfo(cache_dtype).eps
     else:
         assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize("B,Hkv", [(1, 2), (1, 1), (2, 2), (2, 1)])
+@pytest.mark.parametrize("n_hist,T", [(64, 33), (75, 20), (75, 1)])
+def test_attend_chunk_takes_any_layout_of_the_chunk(B, Hkv, n_hist, T):
+    """The chunk's k and v as a model's transposed projections, contiguous per head, or a slice of wider rows: the same
+    bits."""
+    c = kk.KushCache(1, Hkv, 2 * Hkv, 128, batch_size=B, bits=4, device=DEV, dtype=torch.bfloat16)
+    g = torch.Generator().manual_seed(n_hist + T + B)
+    rows = [torch.randn(B, n, 3 * Hkv, 128, generator=g).to(torch.bfloat16).to(DEV) for n in (n_hist, T)]
+    c.write(0, *(rows[0][:, :, i * Hkv:(i + 1) * Hkv].transpose(1, 2) for i in (1, 2)))
+    q = torch.randn(B, 2 * Hkv, T, 128, generator=g).to(torch.bfloat16).to(DEV)
+    wide = [rows[1][:, :, i * Hkv:(i + 1) * Hkv].transpose(1, 2) for i in (1, 2)]
+    per_head = [x.contiguous() for x in wide]
+    projected = [x.transpose(1, 2).contiguous().transpose(1, 2) for x in wide]
+    outs = [c.attend_chunk(0, q, *kv) for kv in (projected, per_head, wide)]
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
