@@ -58,7 +58,7 @@ def _flash(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: bool, scal
     Hk, N = k.shape[1], k.shape[2]
     g = Hq // Hk
     rows = [x.transpose(1, 2) for x in (q, k, v)]
-    if _attend.takes(*rows, scale):
+    if (not causal or N >= T) and _attend.takes(*rows, scale):
         o, lse = _attend.attend(*rows, causal, scale, lse=True)
         return o.transpose(1, 2), lse.transpose(1, 2)
     kt, vt = k.transpose(1, 2).contiguous(), v.transpose(1, 2).contiguous()           # [B, N, Hk, D]
@@ -268,7 +268,7 @@ def unpacked_history_attention(ops, q: torch.Tensor, k_new: torch.Tensor, v_new:
     full = n_hist // PAGE
     r = n_hist - full * PAGE
     key_bytes = 2 * B * Hk * D * (torch.finfo(dt).bits // 8)
-    kernel = T > 0 and q.dtype == dt and fused_ok(q) and _attend.takes(q.transpose(1, 2), *(
+    kernel = k_new.shape[2] == T > 0 and q.dtype == dt and fused_ok(q) and _attend.takes(q.transpose(1, 2), *(
         x.transpose(1, 2) for x in (k_new, v_new)), scale)
     if kernel and n_hist and (n_hist + T) * key_bytes <= block_bytes:
         kp, vp = _unpacked_rows(ops, k_new, v_new, cache, block_table, n_hist, tail_k, tail_idx, rot)

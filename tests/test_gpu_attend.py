@@ -130,6 +130,30 @@ def test_a_prompt_over_keys_of_another_length(N):
     assert got.dtype == q.dtype and _rel(got[0], want) < BOUND[torch.bfloat16]
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("history", [0, 75])
+@pytest.mark.parametrize("N", [20, 50])
+def test_a_chunk_of_more_or_fewer_keys_than_queries(history, N):
+    """attend_chunk where k and v do not hold one row per query: every query sees the whole history, and the chunk's keys
+    up to N - T + t, as before the history and the chunk were attended in one call."""
+    import kushkash_amd as kk
+    torch.manual_seed(history + N)
+    T, H, G = 33, 2, 2
+    c = kk.KushCache(1, H, H * G, 128, bits=8, device=DEV, dtype=torch.bfloat16, rotate=False)
+    hk, hv = torch.zeros(2, H, 0, 128, dtype=torch.float64)
+    if history:
+        c.write(0, *(torch.randn(1, H, history, 128, device=DEV).bfloat16() for _ in range(2)))
+        hk, hv = (x[0].double().cpu() for x in c.dequantize(0))
+    q, k, v = (torch.randn(1, h, n, 128, device=DEV).bfloat16() for h, n in ((H * G, T), (H, N), (H, N)))
+    got = c.attend_chunk(0, q, k, v)[0]
+    keys, vals = (torch.cat([h, x[0].double().cpu()], 1).repeat_interleave(G, 0) for h, x in ((hk, k), (hv, v)))
+    s = q[0].double().cpu() @ keys.transpose(1, 2) * c.scale
+    s[:, :, history:].masked_fill_(torch.arange(N) > torch.arange(T)[:, None] + N - T, -math.inf)
+    want = torch.nan_to_num(torch.softmax(s, -1)) @ vals                # (no key at all: 0)
+    # the blocks' outputs are rounded to bf16 before their merge: one rounding more
+    assert _rel(got, want) < 1.5 * BOUND[torch.bfloat16]
+
+
 @pytest.mark.parametrize("G", [1, 4, 7, 16])
 def test_the_plan_covers_the_keys_and_bounds_its_scratch(G):
     """Whatever the shape: 4 or 8 waves, a split (if any) of at least 12 key tiles that leaves more than one
