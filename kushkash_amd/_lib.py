@@ -74,6 +74,20 @@ def lib() -> ctypes.CDLL:
     return cdll
 
 
+@lru_cache(None)
+def fastcall():
+    """The native host calls (csrc/kush_fastcall.cpp), or None where they are not built: every call then checks its
+    arguments in Python. They hold the library's addresses, so they must be built for its revision."""
+    try:
+        from . import _fastcall
+    except ImportError:
+        return None
+    if getattr(_fastcall, "ABI", None) != ABI_VERSION:
+        raise RuntimeError(f"kushkash_amd: _fastcall.so is for ABI {getattr(_fastcall, 'ABI', None)}, expected {ABI_VERSION}; "
+                           "rebuild it")
+    return _fastcall
+
+
 def call(name: str, *args) -> None:
     """Run one entry point; -1 (unsupported shape) -> ValueError like the reference's CPU path
     (kushkash/_cpu.py:38-40), any other failure -> RuntimeError with the library's message."""

@@ -177,13 +177,9 @@ class Ops:
         # counters of the fused split-K merge: zero at rest (the last workgroup of each (sequence, kv
         # head) resets its own), so one buffer serves every call of this Ops on one stream at a time
         self._sync = torch.zeros(SYNC_SLOTS, dtype=torch.int32, device=self.device)
-        try:
-            from . import _fastcall
-        except ImportError:                                     # not built: every call checks its arguments in Python
-            _fastcall = None
-        self._fast = _fastcall
-        if _fastcall is not None:
-            self._config = _fastcall.make_config(
+        self._fast = _lib.fastcall()
+        if self._fast is not None:
+            self._config = self._fast.make_config(
                 head_dim, bits, group, self._dt, idx, self._sync.data_ptr(),
                 *(_lib.address(n) for n in ("kush_decode_ex", "kush_append_decode", "kush_write_ex")))
 

@@ -36,6 +36,7 @@ CPU_FLAGS = ["-O3", "-std=c++17", "-fPIC", "-shared", "-fopenmp", "-ffp-contract
 # The native host side of the per-step calls (csrc/kush_fastcall.cpp, a Python extension over torch's headers)
 FAST_LIB = PKG / "_fastcall.so"
 FAST_SOURCE = "kush_fastcall.cpp"
+FAST_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-shared"]
 SOURCES = ("kush_capi.hip", "kush_write.hip", "kush_decode.hip", "kush_rotate.hip",
            "kush_unpack.hip", "kush_attend.hip", "kush_decode_inst.hip")
 # the decode kernel instantiations: one object per (input dtype, rot)
@@ -127,7 +128,7 @@ def source_digest(unit: str | None = None) -> str:
         files = sorted(seen)
     for f in files:
         h.update(f.name.encode() + b"\0" + _code(f.read_text()).encode() + b"\0")
-    h.update(repr(CPU_FLAGS if unit == CPU_SOURCE else (FLAGS, units())).encode())
+    h.update(repr({CPU_SOURCE: CPU_FLAGS, FAST_SOURCE: FAST_FLAGS}.get(unit, (FLAGS, units()))).encode())
     return h.hexdigest()[:16]
 
 
@@ -172,8 +173,10 @@ def fastcall_command(out: Path) -> list[str]:
     import sysconfig
 
     import torch
+
+    from ._lib import ABI_VERSION
     base = Path(torch.__file__).resolve().parent
-    return [cxx(), "-O2", "-std=c++17", "-fPIC", "-shared", f"-I{base / 'include'}",
+    return [cxx(), *FAST_FLAGS, f"-DKUSH_FASTCALL_ABI={ABI_VERSION}", f"-I{ROOT / 'include'}", f"-I{base / 'include'}",
             f"-I{base / 'include/torch/csrc/api/include'}", f"-I{sysconfig.get_paths()['include']}",
             f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-o", str(out),
             str(PKG / "csrc" / FAST_SOURCE), f"-L{base / 'lib'}", "-ltorch_python", "-ltorch_cpu", "-lc10"]
@@ -210,7 +213,7 @@ def build(verbose: bool = False, jobs: int | None = None) -> Path:
             os.replace(tmp, dst)
     import json
     DIGEST.write_text(json.dumps({"all": source_digest(),
-                                  **{u: source_digest(u) for u in SOURCES + (FLOOR_SOURCE, CPU_SOURCE)}},
+                                  **{u: source_digest(u) for u in SOURCES + (FLOOR_SOURCE, CPU_SOURCE, FAST_SOURCE)}},
                                  indent=1) + "\n")
     return LIB
 

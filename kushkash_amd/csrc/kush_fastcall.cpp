@@ -12,21 +12,17 @@
 
 #include <cstdint>
 
+#include "kushkash_amd.h"
+
 namespace {
 
 constexpr long NOT_TAKEN = 1;            // the library's codes are 0 or negative
 constexpr int64_t PAGE = 32;
 
-using DecodeFn = int (*)(int, int, int, int, const void*, void*, const void*, int64_t, int64_t, const void*, const int32_t*,
-                         const int32_t*, const int32_t*, int64_t, int32_t, float, int32_t, float*, float*, int32_t, void*,
-                         int32_t, int32_t*, int32_t, const int32_t*, int32_t);
-using AppendDecodeFn = int (*)(int, int, int, int, const void*, void*, void*, int64_t, int64_t, void*, const int32_t*,
-                               const int32_t*, const int32_t*, int64_t, int32_t, float, int32_t, float*, float*, int32_t,
-                               void*, const void*, const void*, int64_t, int64_t, int32_t, int32_t*, int32_t,
-                               const int32_t*, int32_t);
-using WriteFn = int (*)(int, int, int, const void*, const void*, int64_t, int64_t, const int32_t*, const int32_t*,
-                        const int32_t*, const int32_t*, const int32_t*, int32_t, int32_t, void*, int64_t, int64_t, void*,
-                        const int32_t*, int64_t, int32_t, void*, int32_t);
+// The entry points, as the public header declares them: a changed argument list does not compile here
+using DecodeFn = decltype(&kush_decode_ex);
+using AppendDecodeFn = decltype(&kush_append_decode);
+using WriteFn = decltype(&kush_write_ex);
 
 // What one Ops is built for
 struct Config {
@@ -227,5 +223,6 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_fastcall", nullptr, -1, methods, 
 PyMODINIT_FUNC PyInit__fastcall(void) {
     PyObject* m = PyModule_Create(&module);
     if (m) PyModule_AddIntConstant(m, "NOT_TAKEN", NOT_TAKEN);
+    if (m) PyModule_AddIntConstant(m, "ABI", KUSH_FASTCALL_ABI);      // the library's revision it was built for
     return m;
 }

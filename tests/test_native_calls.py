@@ -78,6 +78,34 @@ def library(tmp_path_factory):
     return out
 
 
+def test_an_extension_of_another_abi_is_refused(monkeypatch):
+    """Built for another revision of the library whose addresses it would call: an error that says so, before any call."""
+    import types
+
+    import kushkash_amd
+    from kushkash_amd import _lib
+    for old in (types.SimpleNamespace(), types.SimpleNamespace(ABI=_lib.ABI_VERSION - 1)):
+        monkeypatch.setitem(sys.modules, "kushkash_amd._fastcall", old)
+        monkeypatch.setattr(kushkash_amd, "_fastcall", old, raising=False)
+        _lib.fastcall.cache_clear()
+        with pytest.raises(RuntimeError, match=f"expected {_lib.ABI_VERSION}; rebuild it"):
+            _lib.fastcall()
+    monkeypatch.undo()
+    _lib.fastcall.cache_clear()
+    assert _lib.fastcall() is None or _lib.fastcall().ABI == _lib.ABI_VERSION
+
+
+def test_the_extension_has_a_source_digest():
+    """Its source, the header whose entry points it calls, and its flags decide it; the build records it."""
+    import importlib
+    build = importlib.import_module("kushkash_amd.build")
+    assert build.source_digest(build.FAST_SOURCE) not in (None, build.source_digest(build.CPU_SOURCE))
+    assert build.built_digest(build.FAST_SOURCE) in (None, build.source_digest(build.FAST_SOURCE))
+    seen = set()
+    build._includes(build.PKG / "csrc" / build.FAST_SOURCE, seen)
+    assert {f.name for f in seen} == {build.FAST_SOURCE, "kushkash_amd.h"}
+
+
 def test_tensors_without_storage(library, tmp_path):
     (tmp_path / "calls.py").write_text(SCRIPT)
     r = subprocess.run([sys.executable, str(tmp_path / "calls.py"), str(library)], capture_output=True, text=True, timeout=300)
