@@ -195,7 +195,7 @@ int kush_combine_ex(int head_dim, int group, int dtype, void* out, const float* 
  * reference raises the driver's error string directly (_cuda.py:39-43). */
 const char* kush_last_error(void);
 
-/* ABI revision of this header (8). No reference counterpart. */
+/* ABI revision of this header (9) and of kushkash_amd_attend.h. No reference counterpart. */
 int kush_abi_version(void);
 
 #ifdef __cplusplus

@@ -6,28 +6,15 @@ from __future__ import annotations
 
 import ctypes
 import math
-from functools import lru_cache
 
 import torch
 
 from . import _lib
 
-_P, _I32, _I64, _F = ctypes.c_void_p, ctypes.c_int32, ctypes.c_int64, ctypes.c_float
-# head_dim, dtype, q, k, v, out, lse, strides, cu_q, cu_k, n_q, n_k, total_q, n_seqs, hkv, group, scale, causal,
-# out_f32, waves, chunk, part_o, part_ml, stream
-SIGNATURE = [_I32, _I32, _P, _P, _P, _P, _P, _P, _P, _P, _I32, _I32, _I64, _I32, _I32, _I32, _F, _I32, _I32, _I32,
-             _I32, _P, _P, _P]
 CUS = 256                        # MI355X compute units
 KEYS = 64                        # keys per tile
 PARTIAL_BYTES = 1 << 28          # at most this much scratch for split keys
 _Strides = ctypes.c_int64 * 15
-
-
-@lru_cache(None)
-def _entry():
-    fn = _lib.lib().kush_attend
-    fn.argtypes, fn.restype = SIGNATURE, ctypes.c_int32
-    return fn
 
 
 def _plain(*ts: torch.Tensor) -> bool:
@@ -134,11 +121,11 @@ def attend(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: bool, scal
     rows = -(-(-(-n_k // KEYS)) // chunk) * total * Hq if chunk else 0          # partial rows: every split's
     part = torch.empty(rows * (D + 2), dtype=torch.float32, device=dev) if chunk else None
     with torch.cuda.device(dev):
-        rc = _entry()(D, 1 if q.dtype == torch.float16 else 2, q.data_ptr(), k.data_ptr(), v.data_ptr(),
-                      out.data_ptr(), logs.data_ptr() if lse else None, ctypes.addressof(strides), cq, ck, n_q, n_k,
-                      total, seqs, Hk, group, scale, int(causal), int(lse), waves, chunk,
-                      part.data_ptr() if chunk else None, part.data_ptr() + rows * D * 4 if chunk else None,
-                      torch.cuda.current_stream(dev).cuda_stream)
+        rc = _lib.lib().kush_attend(
+            D, 1 if q.dtype == torch.float16 else 2, q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
+            logs.data_ptr() if lse else None, ctypes.addressof(strides), cq, ck, n_q, n_k, total, seqs, Hk, group, scale,
+            int(causal), int(lse), waves, chunk, part.data_ptr() if chunk else None,
+            part.data_ptr() + rows * D * 4 if chunk else None, torch.cuda.current_stream(dev).cuda_stream)
     if rc:
         raise RuntimeError(f"kush_attend failed ({rc}): {(_lib.lib().kush_last_error() or b'').decode(errors='replace')}")
     return (out, logs) if lse else out

@@ -14,7 +14,7 @@ from pathlib import Path
 import torch   # noqa: F401  -- loads torch's HIP runtime first; the library binds to it (same soname)
 
 LIB = Path(__file__).resolve().parent / "libkushhip.so"
-ABI_VERSION = 8
+ABI_VERSION = 9
 
 _P, _I32, _I64, _F = ctypes.c_void_p, ctypes.c_int32, ctypes.c_int64, ctypes.c_float
 
@@ -56,6 +56,13 @@ SIGNATURES = {
     "kush_last_error": [],
     "kush_abi_version": [],
 }
+# include/kushkash_amd_attend.h
+ATTEND_SIGNATURES = {
+    # head_dim, dtype, q, k, v, out, lse, strides, cu_q, cu_k, n_q, n_k, total_q, n_seqs, hkv, group, scale, causal,
+    # out_f32, waves, chunk, part_o, part_ml, stream
+    "kush_attend": [_I32, _I32, _P, _P, _P, _P, _P, _P, _P, _P, _I32, _I32, _I64, _I32, _I32, _I32, _F, _I32, _I32, _I32,
+                    _I32, _P, _P, _P],
+}
 
 
 @lru_cache(None)
@@ -64,13 +71,13 @@ def lib() -> ctypes.CDLL:
         raise RuntimeError(f"kushkash_amd: {LIB.name} is not built; run `python -m kushkash_amd.build` "
                            "(hipcc, gfx950)")
     cdll = ctypes.CDLL(str(LIB))
-    for name, args in SIGNATURES.items():
+    if cdll.kush_abi_version() != ABI_VERSION:                  # before anything it may not export is looked up
+        raise RuntimeError(f"kushkash_amd: {LIB.name} has ABI {cdll.kush_abi_version()}, expected {ABI_VERSION}; "
+                           "rebuild it")
+    for name, args in (SIGNATURES | ATTEND_SIGNATURES).items():
         fn = getattr(cdll, name)
         fn.argtypes = args
         fn.restype = ctypes.c_char_p if name == "kush_last_error" else ctypes.c_int32
-    if cdll.kush_abi_version() != ABI_VERSION:
-        raise RuntimeError(f"kushkash_amd: {LIB.name} has ABI {cdll.kush_abi_version()}, expected {ABI_VERSION}; "
-                           "rebuild it")
     return cdll
 
 

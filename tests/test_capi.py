@@ -88,6 +88,34 @@ def test_library_exports_every_header_symbol(lib):
     assert set(_lib.SIGNATURES) == set(header_functions())
 
 
+def test_library_exports_the_attend_header(lib):
+    """include/kushkash_amd_attend.h: exported, and bound parameter by parameter as declared."""
+    params = header_params(HEADER.parent / "kushkash_amd_attend.h")
+    assert set(params) == set(_lib.ATTEND_SIGNATURES) == {"kush_attend"}
+    kinds = {"int": ctypes.c_int32, "int32_t": ctypes.c_int32, "int64_t": ctypes.c_int64, "float": ctypes.c_float}
+    for name, decl in params.items():
+        want = [ctypes.c_void_p if "*" in p else kinds[p.split()[0]] for p in decl]
+        assert _lib.ATTEND_SIGNATURES[name] == want and getattr(lib, name).argtypes == want
+
+
+def test_an_older_library_is_refused_by_its_revision(monkeypatch, tmp_path):
+    """One from before the prefill attention, without its entry point: the revision is what is said, not a missing symbol."""
+    class Older:
+        kush_abi_version = staticmethod(lambda: 8)
+
+    fake = tmp_path / "libkushhip.so"
+    fake.write_bytes(b"")
+    monkeypatch.setattr(_lib, "LIB", fake)
+    monkeypatch.setattr(ctypes, "CDLL", lambda path: Older())
+    _lib.lib.cache_clear()
+    try:
+        with pytest.raises(RuntimeError, match=f"has ABI 8, expected {_lib.ABI_VERSION}; rebuild it"):
+            _lib.lib()
+    finally:
+        monkeypatch.undo()
+        _lib.lib.cache_clear()
+
+
 def test_cpu_library_exports_every_cpu_header_symbol():
     """libkushcpu.so (the CPU path) exports what include/kushkash_amd_cpu.h declares, with the parameter
     names and types its binding uses: the reference's CPU ABI (kush/cpu.mojo:476-562) plus one
