@@ -60,7 +60,7 @@ def takes(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: float) -> bo
     return True
 
 
-def plan(spans, group: int, hkv: int, D: int, total_q: int) -> tuple[int, int]:
+def plan(spans, group: int, hkv: int, D: int, total_q: int, causal: bool = True) -> tuple[int, int]:
     """(waves, chunk) of a call whose sequences have (T, N, count) query rows and keys. A row tile is 32 waves
     query rows (group heads of each token) of one kv head; 4 waves fill half a CU (a whole one at D 256, a
     quarter at D 64), 8 a whole one.
@@ -80,7 +80,7 @@ def plan(spans, group: int, hkv: int, D: int, total_q: int) -> tuple[int, int]:
     for t, n, c in spans:
         tiles = -(-t * group // bm) * c
         tasks += tiles
-        units += tiles * -(-(n - t // 2) // KEYS)
+        units += tiles * -(-(n - t // 2 if causal else n) // KEYS)       # (causal: the mean over the rows, N >= T)
     tasks, units = tasks * hkv, units * hkv
     slots = CUS * {64: 4, 128: 2, 256: 1}[D]
     nt = -(-longest // KEYS)
@@ -107,11 +107,11 @@ def attend(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: bool, scal
     if cu is None:
         seqs, n_q, n_k, total = q.shape[0], q.shape[1], k.shape[1], q.shape[0] * q.shape[1]
         cq = ck = None
-        waves, chunk = plan(((n_q, n_k, seqs),), group, Hk, D, total)
+        waves, chunk = plan(((n_q, n_k, seqs),), group, Hk, D, total, causal)
     else:
         cq, ck, n_q, n_k = cu[0].data_ptr(), cu[1].data_ptr(), cu[2], cu[3]
         seqs, total = len(spans), q.shape[0]
-        waves, chunk = plan([(t, n, 1) for t, n in spans], group, Hk, D, total)
+        waves, chunk = plan([(t, n, 1) for t, n in spans], group, Hk, D, total, causal)
     dev = q.device
     if out is None:
         out = torch.empty(q.shape, dtype=torch.float32 if lse else q.dtype, device=dev)

@@ -170,6 +170,13 @@ def test_the_plan_covers_the_keys_and_bounds_its_scratch(G):
     assert _attend.plan(((2048, 34816, 1),), 4, 8, 128, 2048) == (8, 0)
 
 
+@pytest.mark.parametrize("T,N", [(8192, 2016), (4096, 2048), (3000, 1600), (70000, 20000)])
+def test_the_plan_of_an_unmasked_call_counts_every_key(T, N):
+    """Without a mask all rows see all keys, also where there are more rows than keys: row tiles that fill the chip take
+    them whole (8,192 rows over 2,016 keys, 4 x 8 heads: 311 us, 387 with its keys split)."""
+    assert _attend.plan(((T, N, 1),), 4, 8, 128, T, False)[1] == 0
+
+
 def test_kernels_keep_their_wait_states(tmp_path):
     """On the assembly: every read or overwrite of a 32x32x16 MFMA's result waits, on every control-flow path,
     the 12 states that the compiler keeps in straight-line code (a branch join once broke this in the
