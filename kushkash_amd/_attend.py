@@ -64,17 +64,19 @@ def plan(spans, group: int, hkv: int, D: int, total_q: int, causal: bool = True)
     """(waves, chunk) of a call whose sequences have (T, N, count) query rows and keys. A row tile is 32 waves
     query rows (group heads of each token) of one kv head; 4 waves fill half a CU (a whole one at D 256, a
     quarter at D 64), 8 a whole one.
-      8 waves  share each K / V tile among twice the rows: 1,031-1,045 us against 1,066-1,083 at 2,048 tokens x
-               4 heads over 34,816 keys, all of the chip's 256 row tiles of it busy to the end. With fewer or
-               shorter row tiles the last of them leave more of the chip idle than 4 waves do: 171 us against 146 for
-               two first prompts of 3,001 tokens, 293 against 264 for nine chunks over 8,000 keys.
+      8 waves  share each K / V tile among twice the rows, one workgroup to a CU: 1,048 us against 1,097 at 2,048
+               tokens x 4 heads over 34,816 keys (8 kv heads, D 128), 3-7 % less from 16,384 keys on at D 64 and 128;
+               at 8,192 keys between 2 % more and 4 % less, and 6-20 % more at 2,048. Only where the last round of row
+               tiles fills the chip: 3,584 tokens (448 row tiles, 0.88 of two rounds) 1,843 us against 1,996, 3,072
+               (384, 0.75) 1,811 against 1,647, 2,176 (272, 0.53) 1,836 against 1,573.
       chunk    split the keys of a row tile where the row tiles leave the chip idle, into as many parts as fill it
                (256 tokens over 8,000 keys: 167 -> 67 us), or, where the longest would run on alone, into
                halves (the nine chunks: 315 -> 264 us). Not below 24 tiles: the merge launch costs ~4 us, what 3 key
                tiles cost (1,000 tokens over themselves: 27 us whole, 31-34 split)."""
     longest = max(n for _, n, _ in spans)
     bm = 128
-    if D <= 128 and longest >= 16384 and sum(c * (-(-t * group // 256)) for t, _, c in spans) * hkv >= CUS:
+    wide = sum(c * (-(-t * group // 256)) for t, _, c in spans) * hkv                  # row tiles of 8 waves
+    if D <= 128 and longest >= 16384 and wide >= CUS and wide >= 0.8 * CUS * -(-wide // CUS):
         return 8, 0
     tasks = units = 0
     for t, n, c in spans:

@@ -170,6 +170,12 @@ def test_the_plan_covers_the_keys_and_bounds_its_scratch(G):
     assert _attend.plan(((2048, 34816, 1),), 4, 8, 128, 2048) == (8, 0)
 
 
+@pytest.mark.parametrize("T,waves", [(2048, 8), (3584, 8), (4096, 8), (6144, 8), (2049, 4), (2176, 4), (3072, 4), (4352, 4)])
+def test_the_plan_takes_8_waves_for_full_rounds(T, waves):
+    """Over many keys, 8-wave workgroups only where their last round of row tiles fills most of the chip."""
+    assert _attend.plan(((T, 34816, 1),), 4, 8, 128, T)[0] == waves
+
+
 @pytest.mark.parametrize("T,N", [(8192, 2016), (4096, 2048), (3000, 1600), (70000, 20000)])
 def test_the_plan_of_an_unmasked_call_counts_every_key(T, N):
     """Without a mask all rows see all keys, also where there are more rows than keys: row tiles that fill the chip take
