@@ -70,14 +70,20 @@ def plan(spans, group: int, hkv: int, D: int, total_q: int, causal: bool = True)
                tiles fills the chip: 3,584 tokens (448 row tiles, 0.88 of two rounds) 1,843 us against 1,996, 3,072
                (384, 0.75) 1,811 against 1,647, 2,176 (272, 0.53) 1,836 against 1,573.
       chunk    split the keys of a row tile where the row tiles leave the chip idle, into as many parts as fill it
-               (256 tokens over 8,000 keys: 167 -> 67 us), or, where the longest would run on alone, into
-               halves (the nine chunks: 315 -> 264 us). Not below 24 tiles: the merge launch costs ~4 us, what 3 key
-               tiles cost (1,000 tokens over themselves: 27 us whole, 31-34 split)."""
+               (256 tokens over 8,000 keys: 162 -> 68 us), or, where the longest would run on alone, into
+               halves (nine chunks of 61-395 tokens over 800-8,300 keys: 295 -> 268 us), if that gains more than the
+               partials cost: half of what the longest row tile is over an even share (the workgroups left have
+               more of a CU by then; 0.7 at D 256, one workgroup to a CU) against their bytes out and in at 2.5
+               TB/s. The constants are from 700 drawn calls of both sides; without the condition 118 of them were
+               2-32 % slower than whole (3,072 tokens over themselves: 101 -> 129 us, 2,048 at D 64: 43 -> 52), with
+               it 7 (up to 13 %), and 9 of the splits that it leaves out would have gained 2-13 %.
+               Not below 24 tiles (1,000 tokens over themselves: 31 us whole, 31-34 split)."""
     longest = max(n for _, n, _ in spans)
     bm = 128
-    wide = sum(c * (-(-t * group // 256)) for t, _, c in spans) * hkv                  # row tiles of 8 waves
-    if D <= 128 and longest >= 16384 and wide >= CUS and wide >= 0.8 * CUS * -(-wide // CUS):
-        return 8, 0
+    if D <= 128 and longest >= 16384:
+        wide = sum(c * (-(-t * group // 256)) for t, _, c in spans) * hkv              # row tiles of 8 waves
+        if wide >= CUS and wide >= 0.8 * CUS * -(-wide // CUS):
+            return 8, 0
     tasks = units = 0
     for t, n, c in spans:
         tiles = -(-t * group // bm) * c
@@ -85,6 +91,7 @@ def plan(spans, group: int, hkv: int, D: int, total_q: int, causal: bool = True)
         units += tiles * -(-(n - t // 2 if causal else n) // KEYS)       # (causal: the mean over the rows, N >= T)
     tasks, units = tasks * hkv, units * hkv
     slots = CUS * {64: 4, 128: 2, 256: 1}[D]
+    tile_us = {64: 1.26, 128: 2.14, 256: 2.88}[D]                    # a key tile's time with all slots taken
     nt = -(-longest // KEYS)
     if nt < 24 or not tasks:
         return 4, 0
@@ -96,7 +103,10 @@ def plan(spans, group: int, hkv: int, D: int, total_q: int, causal: bool = True)
         return 4, 0
     row = total_q * hkv * group * (D + 2) * 4
     chunk = max(chunk, 12, -(-nt * row // PARTIAL_BYTES))
-    return 4, chunk if chunk < nt else 0
+    gain = (0.7 if D == 256 else 0.5) * (nt - units / slots) * tile_us
+    if chunk >= nt or gain <= -(-nt // chunk) * row * 2 / 2.5e6:
+        return 4, 0
+    return 4, chunk
 
 
 def attend(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: bool, scale: float, lse: bool = False,

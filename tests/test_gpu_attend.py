@@ -170,6 +170,16 @@ def test_the_plan_covers_the_keys_and_bounds_its_scratch(G):
     assert _attend.plan(((2048, 34816, 1),), 4, 8, 128, 2048) == (8, 0)
 
 
+# spans, q heads per kv head, kv heads, D: splitting the keys measured slower than whole, or at least 1.2 times as fast
+@pytest.mark.parametrize("spans,G,hkv,D,split", [
+    ([(2048, 2048, 1)], 4, 8, 128, False), ([(2048, 2048, 1)], 4, 8, 64, False), ([(3072, 3072, 1)], 4, 8, 128, False),
+    ([(1600, 1600, 1)], 4, 8, 256, False), ([(2826, 2826, 4)], 2, 4, 128, False), ([(4225, 4225, 1)], 12, 2, 128, False),
+    ([(256, 8000, 1)], 4, 8, 128, True), ([(512, 34816, 1)], 4, 8, 128, True), ([(1280, 8192, 1)], 4, 8, 64, True),
+    ([(64, 34816, 4)], 4, 8, 128, True), ([(41, 34187, 1)], 7, 1, 128, True), ([(239, 10522, 1)], 4, 8, 256, True), ([(512, 1600, 1)], 4, 8, 256, True)])
+def test_the_plan_splits_keys_where_that_pays(spans, G, hkv, D, split):
+    assert (_attend.plan(spans, G, hkv, D, sum(t * c for t, _, c in spans))[1] > 0) == split
+
+
 @pytest.mark.parametrize("T,waves", [(2048, 8), (3584, 8), (4096, 8), (6144, 8), (2049, 4), (2176, 4), (3072, 4), (4352, 4)])
 def test_the_plan_takes_8_waves_for_full_rounds(T, waves):
     """Over many keys, 8-wave workgroups only where their last round of row tiles fills most of the chip."""
