@@ -113,7 +113,8 @@ def _split_count(sms: int, units: int, pages: int, record: int, chunked: bool) -
     the CUs idle 6 %, and up to 10 % behind the powers of two where those fill the CUs exactly (int4, 8 kv heads,
     4 sequences of 4,096 tokens: 7 splits 14.3 us, 8 splits 13.7; 2 of 131,072: 13 splits 69.9 us, 16 splits 66.6).
     The most that this rule is behind either is 4.4 %.
-    Two at least where they fit: a row's weights are rounded to fp16 relative to the largest of their split and wave,
+    Two at least where they fit (with one workgroup to a CU, 3 pages per wave each: 34 sequences x 2 kv heads of 721
+    tokens, int8, 13.1 us whole, 14.6 in two): a row's weights are rounded to fp16 relative to the largest of their split and wave,
     so fewer splits are less exact (1,000 tokens, fp16: 2.90e-4 from 64 bits at 1 split, 2.71e-4 at 3, 2.62e-4 at 8),
     and one split would save ~1 us of 12 up to 1,000 tokens.
     chunked: past 16 q heads per kv head (two workgroups on each page) powers of two alone (4 x 2 heads of 4,000
@@ -125,7 +126,8 @@ def _split_count(sms: int, units: int, pages: int, record: int, chunked: bool) -
     merge = math.sqrt(4736 / record)
     most = min(256, (sms if single else 2 * sms) // units, pages // (2 * DECODE_WAVES))
     best, least = 1, math.inf
-    for ns in range(2 if most >= 2 and 2 * units <= sms else 1, most + 1):
+    two = most >= 2 and 2 * units <= sms and pages >= (6 if single else 4) * DECODE_WAVES
+    for ns in range(2 if two else 1, most + 1):
         if chunked and ns & (ns - 1):
             continue
         pairs = -(-(-(-pages // ns)) // 2)

@@ -32,7 +32,7 @@ def test_split_policy(D, bits, G):
 @pytest.mark.parametrize("S,H,D,bits,tokens,good", [
     (12, 4, 128, 4, 1000, (2, 3)), (4, 8, 128, 4, 4096, (8,)), (2, 8, 128, 4, 131072, (16,)),
     (1, 8, 128, 4, 131072, (26, 32)), (8, 8, 128, 4, 131072, (3, 4)), (3, 8, 64, 4, 32768, (10, 21)),
-    (2, 8, 64, 4, 65536, (16,)), (1, 4, 256, 8, 4096, (8, 16))])
+    (2, 8, 64, 4, 65536, (16,)), (1, 4, 256, 8, 4096, (8, 16)), (34, 2, 128, 8, 721, (1,))])
 def test_small_batches_fill_the_chip(S, H, D, bits, tokens, good):
     ops = Ops.__new__(Ops)
     ops.D, ops.bits, ops.G, ops.gpu, ops.sms = D, bits, 4, True, 256
