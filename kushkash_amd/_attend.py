@@ -14,7 +14,12 @@ from . import _lib
 CUS = 256                        # MI355X compute units
 KEYS = 64                        # keys per tile
 PARTIAL_BYTES = 1 << 28          # at most this much scratch for split keys
+SLOTS = {64: 4 * CUS, 128: 2 * CUS, 256: CUS}       # 4-wave workgroups the chip holds at once, by head_dim
+TILE_US = {64: 1.26, 128: 2.14, 256: 2.88}          # a key tile's time with all of them taken
 _Strides = ctypes.c_int64 * 15
+# torch.jit.trace, a vmap / grad / functionalize level, and dispatch modes (read on every call)
+_tracing, _transform, _modes = (torch._C._get_tracing_state, torch._C._functorch.peek_interpreter_stack,
+                                torch._C._len_torch_dispatch_stack)
 
 
 def _plain(*ts: torch.Tensor) -> bool:
@@ -24,8 +29,7 @@ def _plain(*ts: torch.Tensor) -> bool:
         return False
     if torch.is_grad_enabled() and any(t.requires_grad for t in ts):
         return False
-    return not (torch.compiler.is_compiling() or torch._C._get_tracing_state() is not None      # (torch.jit.trace)
-                or torch._C._functorch.peek_interpreter_stack() is not None or torch._C._len_torch_dispatch_stack()
+    return not (torch.compiler.is_compiling() or _tracing() is not None or _transform() is not None or _modes()
                 or torch.autograd.forward_ad._current_level >= 0)
 
 
@@ -78,32 +82,30 @@ def plan(spans, group: int, hkv: int, D: int, total_q: int, causal: bool = True)
                2-32 % slower than whole (3,072 tokens over themselves: 101 -> 129 us, 2,048 at D 64: 43 -> 52), with
                it 7 (up to 13 %), and 9 of the splits that it leaves out would have gained 2-13 %.
                Not below 24 tiles (1,000 tokens over themselves: 31 us whole, 31-34 split)."""
-    longest = max(n for _, n, _ in spans)
-    bm = 128
+    longest = max([n for _, n, _ in spans])
+    nt = -(-longest // KEYS)
+    if nt < 24:
+        return 4, 0
     if D <= 128 and longest >= 16384:
         wide = sum(c * (-(-t * group // 256)) for t, _, c in spans) * hkv              # row tiles of 8 waves
         if wide >= CUS and wide >= 0.8 * CUS * -(-wide // CUS):
             return 8, 0
     tasks = units = 0
     for t, n, c in spans:
-        tiles = -(-t * group // bm) * c
+        tiles = -(-t * group // 128) * c
         tasks += tiles
         units += tiles * -(-(n - t // 2 if causal else n) // KEYS)       # (causal: the mean over the rows, N >= T)
     tasks, units = tasks * hkv, units * hkv
-    slots = CUS * {64: 4, 128: 2, 256: 1}[D]
-    tile_us = {64: 1.26, 128: 2.14, 256: 2.88}[D]                    # a key tile's time with all slots taken
-    nt = -(-longest // KEYS)
-    if nt < 24 or not tasks:
+    if not tasks:
         return 4, 0
+    slots = SLOTS[D]
     if 2 * tasks <= slots:
         chunk = -(-nt // (slots // tasks))
-    elif nt * slots > (1.2 if tasks > slots else 1.6) * units:
-        chunk = -(-max(2 * units // slots, nt) // 2)
     else:
-        return 4, 0
+        chunk = -(-max(2 * units // slots, nt) // 2)
     row = total_q * hkv * group * (D + 2) * 4
     chunk = max(chunk, 12, -(-nt * row // PARTIAL_BYTES))
-    gain = (0.7 if D == 256 else 0.5) * (nt - units / slots) * tile_us
+    gain = (0.7 if D == 256 else 0.5) * (nt - units / slots) * TILE_US[D]
     if chunk >= nt or gain <= -(-nt // chunk) * row * 2 / 2.5e6:
         return 4, 0
     return 4, chunk
