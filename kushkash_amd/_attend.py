@@ -64,7 +64,8 @@ def takes(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: float) -> bo
     return True
 
 
-def plan(spans, group: int, hkv: int, D: int, total_q: int, causal: bool = True) -> tuple[int, int]:
+def plan(spans, group: int, hkv: int, D: int, total_q: int, causal: bool = True,
+         scratch: int = PARTIAL_BYTES) -> tuple[int, int]:
     """(waves, chunk) of a call whose sequences have (T, N, count) query rows and keys. A row tile is 32 waves
     query rows (group heads of each token) of one kv head; 4 waves fill half a CU (a whole one at D 256, a
     quarter at D 64), 8 a whole one.
@@ -81,7 +82,8 @@ def plan(spans, group: int, hkv: int, D: int, total_q: int, causal: bool = True)
                TB/s. The constants are from 700 drawn calls of both sides; without the condition 118 of them were
                2-32 % slower than whole (3,072 tokens over themselves: 101 -> 129 us, 2,048 at D 64: 43 -> 52), with
                it 7 (up to 13 %), and 9 of the splits that it leaves out would have gained 2-13 %.
-               Not below 24 tiles (1,000 tokens over themselves: 31 us whole, 31-34 split)."""
+               Not below 24 tiles (1,000 tokens over themselves: 31 us whole, 31-34 split), and into no more parts
+               than min(scratch, PARTIAL_BYTES) holds the partials of."""
     longest = max([n for _, n, _ in spans])
     nt = -(-longest // KEYS)
     if nt < 24:
@@ -104,7 +106,10 @@ def plan(spans, group: int, hkv: int, D: int, total_q: int, causal: bool = True)
     else:
         chunk = -(-max(2 * units // slots, nt) // 2)
     row = total_q * hkv * group * (D + 2) * 4
-    chunk = max(chunk, 12, -(-nt * row // PARTIAL_BYTES))
+    parts = min(scratch, PARTIAL_BYTES) // row                          # at most, in the scratch
+    if parts < 2:
+        return 4, 0
+    chunk = max(chunk, 12, -(-nt // parts))
     gain = (0.7 if D == 256 else 0.5) * (nt - units / slots) * TILE_US[D]
     if chunk >= nt or gain <= -(-nt // chunk) * row * 2 / 2.5e6:
         return 4, 0
@@ -112,20 +117,21 @@ def plan(spans, group: int, hkv: int, D: int, total_q: int, causal: bool = True)
 
 
 def attend(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: bool, scale: float, lse: bool = False,
-           cu: tuple | None = None, spans=None, out: torch.Tensor | None = None):
+           cu: tuple | None = None, spans=None, out: torch.Tensor | None = None, scratch: int = PARTIAL_BYTES):
     """Attention of inputs that takes() accepts: out in q's shape and type (the given one, its rows 16-byte
     aligned, or a new one), or with lse the pair (out fp32, lse fp32 [.., Hq]). cu = (cu_q, cu_k, max_q, max_k)
-    and spans = [(T, N)] for packed rows: the offsets as int32 device tensors, the lengths on the host."""
+    and spans = [(T, N)] for packed rows: the offsets as int32 device tensors, the lengths on the host. scratch: the
+    bytes that partials of split keys may take."""
     D, Hq, Hk = q.shape[-1], q.shape[-2], k.shape[-2]
     group = Hq // Hk
     if cu is None:
         seqs, n_q, n_k, total = q.shape[0], q.shape[1], k.shape[1], q.shape[0] * q.shape[1]
         cq = ck = None
-        waves, chunk = plan(((n_q, n_k, seqs),), group, Hk, D, total, causal)
+        waves, chunk = plan(((n_q, n_k, seqs),), group, Hk, D, total, causal, scratch)
     else:
         cq, ck, n_q, n_k = cu[0].data_ptr(), cu[1].data_ptr(), cu[2], cu[3]
         seqs, total = len(spans), q.shape[0]
-        waves, chunk = plan([(t, n, 1) for t, n in spans], group, Hk, D, total, causal)
+        waves, chunk = plan([(t, n, 1) for t, n in spans], group, Hk, D, total, causal, scratch)
     dev = q.device
     if out is None:
         out = torch.empty(q.shape, dtype=torch.float32 if lse else q.dtype, device=dev)

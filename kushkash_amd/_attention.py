@@ -49,9 +49,10 @@ def fused_ok(q: torch.Tensor) -> bool:
             and _flash_takes(q.dtype, q.shape[-1], q.device))
 
 
-def _flash(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: bool, scale: float):
+def _flash(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: bool, scale: float,
+           block_bytes: int = 1 << 28):
     """attn_lse by the prefill attention kernel, by torch's flash-attention kernel for what that does not
-    take, or None where both refuse the input. torch's: without a mask the q heads of a kv head are folded
+    take, or None where both refuse the input; partials of split keys within block_bytes. torch's: without a mask the q heads of a kv head are folded
     into its query rows (one kernel head per kv head); causal blocks pass the head groups to the kernel,
     which aligns the queries with the last T keys."""
     B, Hq, T, D = q.shape
@@ -59,7 +60,7 @@ def _flash(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: bool, scal
     g = Hq // Hk
     rows = [x.transpose(1, 2) for x in (q, k, v)]
     if (not causal or N >= T) and _attend.takes(*rows, scale):
-        o, lse = _attend.attend(*rows, causal, scale, lse=True)
+        o, lse = _attend.attend(*rows, causal, scale, lse=True, scratch=block_bytes)
         return o.transpose(1, 2), lse.transpose(1, 2)
     kt, vt = k.transpose(1, 2).contiguous(), v.transpose(1, 2).contiguous()           # [B, N, Hk, D]
     try:
@@ -77,20 +78,21 @@ def _flash(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: bool, scal
 
 
 def attn_lse(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: bool, scale: float,
-             key_offset: int | None = None, fused: bool = False) -> tuple[torch.Tensor, torch.Tensor]:
+             key_offset: int | None = None, fused: bool = False,
+             block_bytes: int = 1 << 28) -> tuple[torch.Tensor, torch.Tensor]:
     """(out fp32 [B, Hq, T, D], log-sum-exp fp32 [B, Hq, T]) of q [B, Hq, T, D] over k, v [B, Hk, N, D]
     (GQA: q head i reads kv head i // (Hq / Hk)). The q heads of a kv head are folded into its query
     rows, so K and V are never expanded. causal: query t sees keys j <= key_offset + t (default
     N - T: the queries are the last T of the keys); a query that sees no key gets out 0 and lse -inf
-    (_ops.py:254-276). fused: torch's flash-attention kernel where it takes the input (no mask, or
-    the default causal alignment with N >= T), else the fp32 products."""
+    (_ops.py:254-276). fused: a flash-attention kernel (_flash) where one takes the input (no mask, or
+    the default causal alignment with N >= T), else the fp32 products, in blocks that keep within block_bytes."""
     B, Hq, T, D = q.shape
     Hk, N = k.shape[1], k.shape[2]
     if fused and fused_ok(q) and N > 0 and (not causal or ((key_offset is None or key_offset == N - T) and N >= T)):
-        r = _flash(q, k, v, causal, scale)
+        r = _flash(q, k, v, causal, scale, block_bytes)
         if r is not None:
             return r
-        n = keys_per_block(q, Hk, 2 * B * Hk * D * 4, 1 << 28, 1)     # refused: products, scores bounded
+        n = keys_per_block(q, Hk, 2 * B * Hk * D * 4, block_bytes, 1)     # refused: products, scores bounded
         if not causal and n < N:
             acc = None
             for j0 in range(0, N, n):
@@ -140,7 +142,7 @@ def self_attention_blocks(q: torch.Tensor, k_new: torch.Tensor, v_new: torch.Ten
     T, D = q.shape[2], q.shape[3]
     B, Hk = k_new.shape[0], k_new.shape[1]
     if fused and fused_ok(q) and T > 0:
-        r = _flash(q, k_new, v_new, True, scale)
+        r = _flash(q, k_new, v_new, True, scale, block_bytes)
         if r is not None:
             return merge(acc, r)
     n = keys_per_block(q, Hk, 2 * B * Hk * D * 4, block_bytes, 1)
@@ -166,7 +168,7 @@ def ragged_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, q_start:
         spans = [(b - a, d - c) for a, b, c, d in zip(q_start[:-1], q_start[1:], k_start[:-1], k_start[1:])]
         if _attend.takes(q, k, v, scale) and all(n >= t for t, n in spans):
             dst = out if out is not None and _attend.takes(out, k, v, scale) else None
-            o = _attend.attend(q, k, v, True, scale, cu=varlen, spans=spans, out=dst)
+            o = _attend.attend(q, k, v, True, scale, cu=varlen, spans=spans, out=dst, scratch=block_bytes)
             return o if out is None or dst is not None else out.copy_(o)
         try:
             o = torch.ops.aten._flash_attention_forward(q, k, v, cu_q, cu_k, max_q, max_k, 0.0, True, False,
@@ -259,7 +261,8 @@ def unpacked_history_attention(ops, q: torch.Tensor, k_new: torch.Tensor, v_new:
     rounding to the cache dtype; rot rotates a rotated cache's rows back, so the attention runs on the
     unrotated q and chunk), the partial page's K from the tail slots tail_idx. Where the prefill attention
     kernel takes q, the history and the chunk are unpacked into one set of rows if block_bytes hold them, and
-    attended by one causal call; else each block is attended by itself and the blocks merged. Shapes as
+    attended by one causal call; else each block is attended by itself and the blocks merged. Partials of keys that
+    the kernel splits over the chip keep within block_bytes too. Shapes as
     history_attention; returns [B, Hq, T, D] in q's dtype."""
     B, Hq, T, D = q.shape
     Hk = k_new.shape[1]
@@ -272,9 +275,10 @@ def unpacked_history_attention(ops, q: torch.Tensor, k_new: torch.Tensor, v_new:
         x.transpose(1, 2) for x in (k_new, v_new)), scale)
     if kernel and n_hist and (n_hist + T) * key_bytes <= block_bytes:
         kp, vp = _unpacked_rows(ops, k_new, v_new, cache, block_table, n_hist, tail_k, tail_idx, rot)
-        return _attend.attend(q.transpose(1, 2), kp, vp, True, scale).transpose(1, 2)
+        return _attend.attend(q.transpose(1, 2), kp, vp, True, scale, scratch=block_bytes).transpose(1, 2)
     if kernel and not n_hist:
-        return _attend.attend(*(x.transpose(1, 2) for x in (q, k_new, v_new)), True, scale).transpose(1, 2)
+        rows = [x.transpose(1, 2) for x in (q, k_new, v_new)]
+        return _attend.attend(*rows, True, scale, scratch=block_bytes).transpose(1, 2)
     if n_hist:
         fused = fused_ok(q)
         step = keys_per_block(q, Hk, key_bytes if kernel else key_bytes + 8 * B * Hk * D, block_bytes, PAGE,
@@ -303,7 +307,7 @@ def unpacked_history_attention(ops, q: torch.Tensor, k_new: torch.Tensor, v_new:
             n = (p1 - p0) * PAGE + (r if tail else 0)
             k = kp.view(B, rows, Hk, D)[:, :n].transpose(1, 2)
             v = vp.view(B, rows, Hk, D)[:, :n].transpose(1, 2)
-            acc = merge(acc, attn_lse(q, k, v, False, scale, fused=True))
+            acc = merge(acc, attn_lse(q, k, v, False, scale, fused=True, block_bytes=block_bytes))
             p0 = p1 + (1 if tail else 0)
     acc = self_attention_blocks(q, k_new.to(q.dtype), v_new.to(q.dtype), scale, block_bytes, acc, fused=True)
     return acc[0].to(q.dtype)

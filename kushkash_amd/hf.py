@@ -143,7 +143,7 @@ def prompt_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: f
     transposed views) is never taken either."""
     rows = [x.transpose(1, 2) for x in (q, k, v)]
     if k.shape[2] == q.shape[2] and _attend.takes(*rows, scale):     # else query t sees keys 0 .. t all the same
-        return _attend.attend(*rows, True, scale).transpose(1, 2)
+        return _attend.attend(*rows, True, scale, scratch=block_bytes).transpose(1, 2)
     if q.dtype in (torch.float16, torch.bfloat16):
         g = q.shape[1] // k.shape[1]
         ke = k.repeat_interleave(g, 1) if g > 1 else k

@@ -180,6 +180,49 @@ def test_the_plan_splits_keys_where_that_pays(spans, G, hkv, D, split):
     assert (_attend.plan(spans, G, hkv, D, sum(t * c for t, _, c in spans))[1] > 0) == split
 
 
+def test_the_plan_keeps_its_partials_within_the_scratch():
+    """Every part's rows together within PARTIAL_BYTES, and within what the caller gives where that is less."""
+    split = 0
+    for D in (64, 128, 256):
+        for G, hkv in ((1, 1), (4, 8), (16, 2)):
+            for T in (1, 16, 100, 256, 500, 700, 1100):
+                for N in (1600, 8000, 34816, 200000):
+                    for c in (1, 3):
+                        for scratch in (1 << 30, 1 << 28, 1 << 24, 1 << 20, 0):
+                            waves, chunk = _attend.plan(((T, N, c),), G, hkv, D, T * c, False, scratch)
+                            parts = -(-(-(-N // 64)) // chunk) if chunk else 0
+                            assert parts * T * c * hkv * G * (D + 2) * 4 <= min(scratch, _attend.PARTIAL_BYTES)
+                            split += parts > 1
+    assert split > 100
+    # one long sequence among many rows: half its keys' partials are 1.2 times the bound
+    assert _attend.plan([(1000, 40000, 1), (1000, 1000, 9)], 4, 8, 128, 10000) == (4, 0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("what", ["chunk", "first chunk", "prompt"])
+def test_split_keys_within_block_bytes(what, monkeypatch):
+    """The callers' memory bound reaches the plan: no partials past it, and the answer stays."""
+    import kushkash_amd as kk
+    from kushkash_amd.hf import prompt_attention
+    torch.manual_seed(2)
+    T = 512 if what == "chunk" else 1700
+    q, k, v = (torch.randn(1, h, T, 128, device=DEV).bfloat16() for h in (8, 2, 2))
+    c = kk.KushCache(1, 2, 8, 128, bits=8, device=DEV, dtype=torch.bfloat16)
+    if what == "chunk":
+        c.write(0, *(torch.randn(1, 2, 4096, 128, device=DEV).bfloat16() for _ in range(2)))
+    plans = []
+    real = _attend.plan
+    monkeypatch.setattr(_attend, "plan", lambda *a: plans.append((a, real(*a))) or plans[-1][1])
+    outs = []
+    for bound in (1 << 28, 1 << 22):
+        plans.clear()
+        outs.append(prompt_attention(q, k, v, 0.09, bound) if what == "prompt" else c.attend_chunk(0, q, k, v, bound))
+        for a, (waves, chunk) in plans:
+            nt = -(-max(n for _, n, _ in a[0]) // 64)
+            assert (-(-nt // chunk) if chunk else 0) * a[4] * 8 * 130 * 4 <= bound and plans
+    assert _rel(outs[0], outs[1].double().cpu()) < 3 * BOUND[torch.bfloat16]
+
+
 @pytest.mark.parametrize("T,waves", [(2048, 8), (3584, 8), (4096, 8), (6144, 8), (2049, 4), (2176, 4), (3072, 4), (4352, 4)])
 def test_the_plan_takes_8_waves_for_full_rounds(T, waves):
     """Over many keys, 8-wave workgroups only where their last round of row tiles fills most of the chip."""
