@@ -195,7 +195,7 @@ def test_the_plan_keeps_its_partials_within_the_scratch():
                             split += parts > 1
     assert split > 100
     # one long sequence among many rows: half its keys' partials are 1.2 times the bound
-    assert _attend.plan([(1000, 40000, 1), (1000, 1000, 9)], 4, 8, 128, 10000) == (4, 0)
+    assert _attend.plan([(1000, 15000, 1), (1000, 1000, 9)], 4, 8, 128, 10000) == (4, 0)
 
 
 @pytest.mark.gpu
