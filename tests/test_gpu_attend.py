@@ -94,6 +94,70 @@ def test_inputs_left_to_the_other_paths():
         assert _attend.takes(q, k, v, 0.1)
 
 
+def _same(got, want, bound):
+    """NaN in the same places, the rest within the bound."""
+    got = got.double().cpu()
+    assert torch.equal(got.isnan(), want.isnan())
+    at = ~want.isnan()
+    assert not at.any() or ((got[at] - want[at]).norm() / want[at].norm()).item() < bound
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("waves,chunk", [(4, 0), (8, 0), (4, 1), (8, 2)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("what", ["nan key", "inf key", "-inf keys", "no finite score", "nan query", "nan value"])
+def test_values_that_are_not_finite(what, dtype, waves, chunk, monkeypatch):
+    """Causal, 150 queries over 200 keys: a NaN score makes the rows that see it NaN and no other, +inf too, -inf scores
+    weigh nothing, a row of nothing else is NaN with log-sum-exp -inf, and a query's NaN stays in its row."""
+    torch.manual_seed(11)
+    T, N, Hk, G, D, scale = 150, 200, 2, 2, 128, 0.09
+    q, k, v = (torch.randn(1, n, h, D, device=DEV).to(dtype) for n, h in ((T, Hk * G), (N, Hk), (N, Hk)))
+    q[..., 5] = q[..., 5].abs() + 0.5                                   # an infinite k[..., 5] gives scores of its sign
+    if what == "nan key":
+        k[:, 130, 1, 7] = math.nan
+    elif what == "inf key":
+        k[:, 130, 1, 5] = math.inf
+    elif what == "-inf keys":
+        k[:, 20:128, 0, 5] = -math.inf                                  # a whole key tile among them
+    elif what == "no finite score":
+        k[:, :, 0, 5] = -math.inf
+    elif what == "nan query":
+        q[:, 77, 3, 64] = math.nan
+    else:
+        v[:, 190, 0, 3] = math.nan
+    monkeypatch.setattr(_attend, "plan", lambda *a: (waves, chunk))
+    out = _attend.attend(q, k, v, True, scale)
+    out32, lse = _attend.attend(q, k, v, True, scale, lse=True)
+    want, logs = _exact(q[0], k[0], v[0], True, scale)
+    if what == "nan value":
+        # the product of a zero weight and NaN is NaN: what rows that do not see the key hold is not defined (a tile's
+        # rows have it, others not); those that see it are NaN in that dim, and all other dims are whole
+        assert out[0, 140:, :G, 3].isnan().all()
+        keep = [d for d in range(D) if d != 3]
+        out, out32, want = out[..., keep], out32[..., keep], want[..., keep]
+    _same(out[0], want, BOUND[dtype])
+    _same(out32[0], want, BOUND[dtype])
+    finite = logs.isfinite()
+    # (of a row with a +inf score, whose output is NaN, the kernel's is inf - inf, 64 bits' is inf: neither is used)
+    assert torch.equal(lse[0].cpu().isfinite(), finite) and torch.equal(lse[0].cpu() == -math.inf, logs == -math.inf)
+    assert (lse[0].double().cpu()[finite] - logs[finite]).abs().max() < BOUND[dtype]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dims", [(2,), (0,), (0, 2)])
+def test_rows_that_repeat_over_heads_or_batches(dims):
+    """k and v expanded over heads or batches (strides of 0), and q over batches."""
+    torch.manual_seed(12)
+    B, T, N, Hk, G, D, scale = 3, 70, 130, 2, 3, 64, 0.1
+    q = torch.randn(1 if 0 in dims else B, T, Hk * G, D, device=DEV).bfloat16().expand(B, -1, -1, -1)
+    k, v = (torch.randn(*(1 if i in dims else n for i, n in enumerate((B, N, Hk))), D, device=DEV).bfloat16().expand(B, N, Hk, D)
+            for _ in range(2))
+    assert _attend.takes(q, k, v, scale)
+    out = _attend.attend(q, k, v, True, scale)
+    for b in range(B):
+        assert _rel(out[b], _exact(q[b], k[b], v[b], True, scale)[0]) < BOUND[torch.bfloat16]
+
+
 def test_a_trace_is_not_plain():
     """torch.jit.trace records torch's operators only: under it nothing is the kernel's."""
     x, seen = torch.randn(2, 4), []
