@@ -121,8 +121,9 @@ int kush_decode(int head_dim, int bits, int group, int dtype, const void* q, voi
  *   runs fewer). Every choice is deterministic: the same call gives the same bits.
  * seq_order: NULL, or int32 [n_seqs] holding a permutation of the sequences: their workgroups start
  *   in that order (longest first balances a ragged batch); the results do not depend on it.
- * rot: 1 for a cache written with rot = 1: q is rotated by the canonical Walsh-Hadamard transform
- *   (rounded to dtype, as kush_fwht) on load and the output rotated back before its one rounding to
+ * rot: 1 for a cache written with rot = 1: q is rotated by the Walsh-Hadamard transform, rounded to dtype,
+ *   on load (fp32 in kush_fwht's order; fp16 and bf16 with its fp32 sums in another order, so that a value on
+ *   the edge of a rounding may go the other way) and the output rotated back before its one rounding to
  *   dtype; the split partials stay unrotated (kush_combine_ex takes the same rot). */
 int kush_decode_ex(int head_dim, int bits, int group, int dtype, const void* q, void* out, const void* cache,
                    int64_t block_stride, int64_t head_stride, const void* tail_k, const int32_t* tail_idx,

@@ -52,9 +52,9 @@ def fused_ok(q: torch.Tensor) -> bool:
 def _flash(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: bool, scale: float,
            block_bytes: int = 1 << 28):
     """attn_lse by the prefill attention kernel, by torch's flash-attention kernel for what that does not
-    take, or None where both refuse the input; partials of split keys within block_bytes. torch's: without a mask the q heads of a kv head are folded
-    into its query rows (one kernel head per kv head); causal blocks pass the head groups to the kernel,
-    which aligns the queries with the last T keys."""
+    take, or None where both refuse the input; partials of split keys within block_bytes. torch's: without a
+    mask the q heads of a kv head are folded into its query rows (one kernel head per kv head); causal blocks
+    pass the head groups to the kernel, which aligns the queries with the last T keys."""
     B, Hq, T, D = q.shape
     Hk, N = k.shape[1], k.shape[2]
     g = Hq // Hk

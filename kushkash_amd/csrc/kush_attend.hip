@@ -18,8 +18,9 @@
 //     torch's flash kernel's (1.84e-3 against 1.85e-3 at N(0, 2^2) keys, bf16); moving the max only when it
 //     grows by 2^8 is 3 % faster and 10 % further off, and not taken.
 //   - Two waves per SIMD (8 waves at D <= 128): one's exponentials run under the other's MFMAs.
-// Measured (bf16, causal): 2,048 tokens x 32 heads over 34,816 keys x 8 kv heads, D 128: 1,061-1,118 us,
-// 1,016-1,060 TFLOP/s, where a large bf16 matrix product reaches 1,369 and torch's flash kernel 468.
+// Measured (bf16, causal, device events): 2,048 tokens x 32 heads over 34,816 keys x 8 kv heads, D 128: 1,048 us,
+// 1,082 TFLOP/s (1,081 us, 1,049 TFLOP/s on another card), where a large bf16 matrix product reaches 1,369 and torch's
+// flash kernel 468.
 #include <cmath>
 
 #include "kush_common.h"

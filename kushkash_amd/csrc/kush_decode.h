@@ -261,7 +261,8 @@ __device__ __forceinline__ v2i gather_vt(const uint8_t* slot, int ct, int lane) 
 // V columns gathered ahead of a page pair's softmax: with one wave per SIMD nothing else covers an LDS read's
 // latency, and the compiler, short of registers, read the columns one by one with a full wait behind each.
 // As many as fit the 256 registers beside the loop's own: 4 columns of a pair (16 registers) at D <= 128, 2 of its
-// int8 codes, none with a third pair or a split's folded state beside those, nor at D 256.
+// int8 codes, none with a third pair or a split's folded state beside those, nor at D 256. Without any -> with: 33
+// ragged sequences of D 64, int8, 18.1 -> 17.8 us, one of 333 tokens 9.14 -> 9.00, 64 of 4,096 34.51 -> 34.36.
 template <int D, int BITS, int DEP, bool WS>
 constexpr int vpre() {
     return D == 256 || DEP == 3 || (D == 128 && BITS == 8 && WS) ? 0 : (D == 128 && BITS == 8 ? 2 : 4);
@@ -739,7 +740,8 @@ __device__ __forceinline__ void store_rotated_rows(IN* __restrict__ out, const f
     }
 }
 
-// The staged rows r < n, a wave per row.
+// The staged rows r < n, a wave per row. Against 16 values per lane (fwht_runs): one sequence of 333 tokens, 8 kv
+// heads, 9.4 -> 9.0 us, 4 of 1,000 12.5 -> 12.2; 19 sequences of D 256 with 16 heads per kv head 32.75 -> 33.05.
 template <int D, typename IN, int THREADS>
 __device__ __forceinline__ void store_rotated(IN* __restrict__ out, const float* stage, int n, bool vec) {
     constexpr int NR = THREADS / WAVE;
@@ -755,7 +757,8 @@ __device__ __forceinline__ void store_rotated(IN* __restrict__ out, const float*
 // disjoint groups of index bits (j, lane group, kk), so H = H_8 (x) H_4 (x) H_KS: one MFMA per K-step and row half
 // sums over j and the lane groups with signs +-1 (exact products, fp32 sums; output row 4 q' + i of half hf
 // stands for j = 4 hf + i of lane group q'), and a butterfly over the K-steps in registers does the rest. No LDS
-// and no barrier, where the rotation through LDS put two of each before the second page pair.
+// and no barrier, where the rotation through LDS put two of each before the second page pair: one sequence of 333
+// tokens, 8 kv heads, 9.6 -> 9.0 us; 19 sequences of D 256 with 16 heads per kv head 36.5 -> 33.1.
 template <int D, typename IN>
 __device__ __forceinline__ void rotate_q(const u4 (&qraw)[D / 32], float (&qv)[D / 32][8], int lane) {
     constexpr int KS = D / 32;
@@ -803,7 +806,8 @@ __device__ __forceinline__ void rotate_q(const u4 (&qraw)[D / 32], float (&qv)[D
 // D / 64 dims from l D / 64), rotates them when the cache does, and stores the K row into the tail and the
 // quantized V row into the record -- page_task's arithmetic, so its bytes -- with a copy of both in LDS. The
 // workgroup's own use of the row (its exact score, its V codes) takes those copies, so nothing in the launch
-// waits for the stores, and the page loop starts without the append.
+// waits for the stores, and the page loop starts without the append: one sequence of 333 tokens, 8 kv heads, 10.5 ->
+// 9.0 us, 33 ragged ones of D 64, int8, 18.5 -> 17.6, 19 of D 256 34.1 -> 33.1 (a decode alone of 4 x 1,000: 12.0 -> 12.2).
 template <int D, int BITS, typename IN>
 struct NewToken {
     using F = Fmt<D, BITS>;
@@ -1060,7 +1064,7 @@ __device__ void merge_splits(const float* __restrict__ part_ml, const float* __r
 }
 
 // grid (S, Hkv, n_splits * ceil(G / 16)), block NW * 64. Registers are budgeted for two waves per SIMD
-// (amdgpu_waves_per_eu(2); the library is built with MFMA accumulators in VGPRs): with a 512-register
+// (amdgpu_waves_per_eu(2); naming a maximum too changes no instruction; the library is built with MFMA accumulators in VGPRs): with a 512-register
 // budget the 4-wave variant used 236 VGPRs + 76 AGPRs and spent 46 v_accvgpr moves per page in its
 // loop; at <= 256 it needs none, and two 4-wave workgroups fit on one CU. ST = 2 (G <= 8): two page streams share the
 // MFMA columns (page A of each pair in columns 0-7, page B in 8-15); ST = 1: one page's 16 heads.
@@ -1196,8 +1200,8 @@ __global__ __launch_bounds__(NW * WAVE) __attribute__((amdgpu_waves_per_eu(2, D 
     // head). A token that completes its page goes first: the split that holds the page quantizes it, and its stores
     // are complete and visible to its own page loads after the barrier. Else (31 tokens of 32) the last split,
     // which takes the partial page, appends it behind its first page loads (NewToken). No other workgroup reads
-    // that page or the sequence's tail. One sequence of 333 tokens, 8 kv heads, rotated:
-    // 11.6 -> 9.1 us with rotate_q and the wave-wide output rotation; 200 sequences of 100-200 tokens: 34.7 -> 29.4 us.
+    // that page or the sequence's tail. With rotate_q and the wave-wide output rotation, one sequence of 333 tokens, 8 kv
+    // heads, takes 9.0 us in place of 11.6, and 200 sequences of 100-200 tokens 29.4 in place of 34.7.
     bool appends = false;                                          // this workgroup holds the new token of a partial page
     if (app_k != nullptr && gc == 0 && n > 0) {
         const int pos = n - 1, slot = pos % PAGE, pg = pos / PAGE;
@@ -1388,7 +1392,8 @@ __global__ __launch_bounds__(NW * WAVE) __attribute__((amdgpu_waves_per_eu(2, D 
         if constexpr (RLDS) {
             __syncthreads();                                     // every wave done with the staged q
             KUSH_ISSUE_PAIR(sl2, sl3, pb)
-        }        // One pair step: the pair has landed once at most the other pair's loads are outstanding;
+        }
+        // One pair step: the pair has landed once at most the other pair's loads are outstanding;
         // scores of both pages (the next pair's table read hides behind them), one softmax update,
         // PV of both; then, every read of the
         // two slots complete (lgkmcnt 0), they take the next pair. The second page of a window's odd

@@ -11,10 +11,11 @@ with the same k and v tensors. KushHFCache.update stores nothing; it attaches a 
 layer) -- to the key tensor, and the attention function reads the route off the key it receives. No
 state outlives the call: a forward without a KushHFCache carries no route and is refused. The
 attention function then picks by the chunk length T and the tokens n already cached:
-    T = 1          append the token and decode, one kernel launch (KushCache.append_attend);
+    T = 1          append the token and decode (KushCache.append_attend);
     T > 1, n = 0   causal attention over the prompt itself, then the chunk write;
-    T > 1, n > 0   attention over the history (unpacked a block at a time by the unpack kernel) and
-                   the chunk (causal), merged by log-sum-exp (KushCache.attend_chunk); then the write.
+    T > 1, n > 0   attention over the history (unpacked by the unpack kernel) and the chunk (causal), as one
+                   set of rows or a block of history at a time, merged by log-sum-exp (KushCache.attend_chunk);
+                   then the write.
 """
 from __future__ import annotations
 
@@ -137,10 +138,10 @@ def prompt_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: f
     [B, Hkv, T, D] -> [B, Hq, T, D] in q's dtype (hf.py:122-129). Half-precision inputs go to the prefill
     attention kernel; what it does not take (rows not 16-byte aligned, derivatives) to torch's fused
     attention, limited to its flash kernel (K / V expanded to the q heads); everything else, and any input
-    the flash kernel refuses, to fp32 products over blocks of keys whose memory stays within block_bytes. torch's memory-efficient kernel is not allowed: on ROCm its dense and varlen forms are
-    the same kernel family, and its varlen form with a bottom-right causal mask has taken an
-    illegal-address fault on this device. torch's half-precision math path (batched products over
-    transposed views) is never taken either."""
+    the flash kernel refuses, to fp32 products over blocks of keys whose memory stays within block_bytes.
+    torch's memory-efficient kernel is not allowed: on ROCm its dense and varlen forms are the same kernel
+    family, and its varlen form with a bottom-right causal mask has taken an illegal-address fault on this
+    device. torch's half-precision math path (batched products over transposed views) is never taken either."""
     rows = [x.transpose(1, 2) for x in (q, k, v)]
     if k.shape[2] == q.shape[2] and _attend.takes(*rows, scale):     # else query t sees keys 0 .. t all the same
         return _attend.attend(*rows, True, scale, scratch=block_bytes).transpose(1, 2)
