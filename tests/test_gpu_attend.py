@@ -158,6 +158,27 @@ def test_rows_that_repeat_over_heads_or_batches(dims):
         assert _rel(out[b], _exact(q[b], k[b], v[b], True, scale)[0]) < BOUND[torch.bfloat16]
 
 
+@pytest.mark.gpu
+def test_split_keys_in_a_captured_graph():
+    """A call whose keys are split (partials from the allocator, a second launch), replayed on new inputs with eager work
+    between: the eager call's bits each time."""
+    torch.manual_seed(13)
+    T, N, Hk, G, D, scale = 40, 4000, 2, 4, 128, 0.09
+    rows = [torch.randn(1, n, h, D, device=DEV).bfloat16() for n, h in ((T, Hk * G), (N, Hk), (N, Hk))]
+    assert _attend.plan(((T, N, 1),), G, Hk, D, T)[1] > 0
+    _attend.attend(*rows, True, scale)
+    graph, stream = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    with torch.cuda.graph(graph, stream=stream):
+        out = _attend.attend(*rows, True, scale)
+    for _ in range(4):
+        for x in rows:
+            x.copy_(torch.randn_like(x))
+        want = _attend.attend(*rows, True, scale)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+
+
 def test_a_trace_is_not_plain():
     """torch.jit.trace records torch's operators only: under it nothing is the kernel's."""
     x, seen = torch.randn(2, 4), []
